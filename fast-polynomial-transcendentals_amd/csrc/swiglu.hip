@@ -27,19 +27,58 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv f) {
     return (__umulhi(n, f.m) + n) >> f.l;
 }
 
-// Packed forward: vector v of the output row-major [rows, H] maps to
-// gate vector r*2*hv + c and up vector r*2*hv + hv + c (hv = H/8 vectors).
+// Packed rows at any even H >= 8: a row of H outputs is covered by
+// nv = ceil(H / 8) vectors of 8, vector k at column min(8 k, H - 8), so where
+// H is no multiple of 8 the last vector of a row overlaps the one before it
+// and both store the same values to the columns they share.  Every 16-byte
+// access starts at an even element of 4-byte aligned storage, which global
+// memory takes at full width; a wavefront still covers 1 KiB runs of each
+// stream.  HBM- or MALL-bound like the aligned rows (which are the same code
+// with no overlap).  At 3001 x 2730 BF16, one element per thread, as rows of
+// such widths ran before: forward 18.2, backward 20.6 us; this way 9.5 and
+// 14.4 us.
+typedef u32x4_t u32x4_a4_t __attribute__((aligned(4)));
+
+template <bool NT>
+__device__ __forceinline__ Vec4 ld16_a4(const void* base, int64_t e) {
+    const u32x4_a4_t* p = reinterpret_cast<const u32x4_a4_t*>(reinterpret_cast<const uint16_t*>(base) + e);
+    const u32x4_a4_t v = NT ? __builtin_nontemporal_load(p) : *p;
+    return Vec4{{v.x, v.y, v.z, v.w}};
+}
+
+template <bool NT>
+__device__ __forceinline__ void st16_a4(void* base, int64_t e, const Vec4& v) {
+    u32x4_a4_t* p = reinterpret_cast<u32x4_a4_t*>(reinterpret_cast<uint16_t*>(base) + e);
+    const u32x4_a4_t u = {v.w[0], v.w[1], v.w[2], v.w[3]};
+    if constexpr (NT) {
+        __builtin_nontemporal_store(u, p);
+    } else {
+        *p = u;
+    }
+}
+
+struct PackedShape {
+    uint32_t n_vec, nv, h;  // rows * nv vectors, vectors per row, hidden size
+    FastDiv div_nv;
+    // output element and gate element of vector v (up: + h)
+    __device__ __forceinline__ void at(uint32_t v, int64_t& e, int64_t& g) const {
+        const uint32_t r = fast_div(v, div_nv), c8 = (v - r * nv) * 8;
+        const uint32_t c = c8 < h - 8 ? c8 : h - 8;
+        e = (int64_t)r * h + c;
+        g = e + (int64_t)r * h;
+    }
+};
+
 template <class Op, bool LNT, bool SNT>
 __global__ void __launch_bounds__(kBlock)
-packed_fwd_kernel(const void* __restrict__ packed, void* __restrict__ out, uint32_t n_vec,
-                  uint32_t hv, FastDiv div_hv) {
+packed_fwd_kernel(const void* __restrict__ packed, void* __restrict__ out, PackedShape sh) {
     static_assert(Op::NIN == 2 && Op::NOUT == 1, "packed forward op shape");
     const uint32_t stride = gridDim.x * kBlock;
-    for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n_vec; v += stride) {
-        const uint32_t r = fast_div(v, div_hv);
-        const int64_t g = (int64_t)r * hv + v;  // = r*2*hv + c
-        const Vec4 gate = ld16<LNT>(packed, g);
-        const Vec4 up = ld16<LNT>(packed, g + hv);
+    for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < sh.n_vec; v += stride) {
+        int64_t e, g;
+        sh.at(v, e, g);
+        const Vec4 gate = ld16_a4<LNT>(packed, g);
+        const Vec4 up = ld16_a4<LNT>(packed, g + sh.h);
         Vec4 o;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -47,7 +86,7 @@ packed_fwd_kernel(const void* __restrict__ packed, void* __restrict__ out, uint3
             Op::pair(a, b);
             o.w[w] = b[0];
         }
-        st16<SNT>(out, v, o);
+        st16_a4<SNT>(out, e, o);
     }
 }
 
@@ -55,15 +94,15 @@ packed_fwd_kernel(const void* __restrict__ packed, void* __restrict__ out, uint3
 template <class Op, bool LNT, bool SNT>
 __global__ void __launch_bounds__(kBlock)
 packed_bwd_kernel(const void* __restrict__ grad_out, const void* __restrict__ packed,
-                  void* __restrict__ grad_packed, uint32_t n_vec, uint32_t hv, FastDiv div_hv) {
+                  void* __restrict__ grad_packed, PackedShape sh) {
     static_assert(Op::NIN == 3 && Op::NOUT == 2, "packed backward op shape");
     const uint32_t stride = gridDim.x * kBlock;
-    for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < n_vec; v += stride) {
-        const uint32_t r = fast_div(v, div_hv);
-        const int64_t g = (int64_t)r * hv + v;
-        const Vec4 go = ld16<LNT>(grad_out, v);
-        const Vec4 gate = ld16<LNT>(packed, g);
-        const Vec4 up = ld16<LNT>(packed, g + hv);
+    for (uint32_t v = blockIdx.x * kBlock + threadIdx.x; v < sh.n_vec; v += stride) {
+        int64_t e, g;
+        sh.at(v, e, g);
+        const Vec4 go = ld16_a4<LNT>(grad_out, e);
+        const Vec4 gate = ld16_a4<LNT>(packed, g);
+        const Vec4 up = ld16_a4<LNT>(packed, g + sh.h);
         Vec4 gg, gu;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -72,12 +111,12 @@ packed_bwd_kernel(const void* __restrict__ grad_out, const void* __restrict__ pa
             gg.w[w] = b[0];
             gu.w[w] = b[1];
         }
-        st16<SNT>(grad_packed, g, gg);
-        st16<SNT>(grad_packed, g + hv, gu);
+        st16_a4<SNT>(grad_packed, g, gg);
+        st16_a4<SNT>(grad_packed, g + sh.h, gu);
     }
 }
 
-// Element path (H not a multiple of 8, unaligned storage or > 2^31 vectors).
+// Element path (odd H or H < 8, storage not 4-byte aligned, or >= 2^31 vectors).
 template <class Op, bool BWD>
 __global__ void __launch_bounds__(kBlock)
 packed_element_kernel(const void* __restrict__ grad_out, const void* __restrict__ packed,
@@ -111,17 +150,17 @@ int launch_packed(void* out, const void* grad_out, const void* packed, int64_t r
     const int64_t n = rows * h;
     if (n == 0) return hipSuccess;
     if (!out || !packed || (BWD && !grad_out)) return hipErrorInvalidValue;
-    const int64_t n_vec = n / 8;
-    const bool vec = (h % 8 == 0) && aligned16(out) && aligned16(packed) &&
-                     (!BWD || aligned16(grad_out)) && n_vec < (int64_t(1) << 31);
+    const auto aligned4 = [](const void* p) { return ((uintptr_t)p & 3u) == 0; };
+    const int64_t nv = (h + 7) / 8, n_vec = rows * nv;
+    const bool vec = h % 2 == 0 && h >= 8 && aligned4(out) && aligned4(packed) && (!BWD || aligned4(grad_out)) &&
+                     n_vec < (int64_t(1) << 31) && h < (int64_t(1) << 31);
     if (!vec) {
         const int64_t grid = grid_one_pass(n);
         hipLaunchKernelGGL((packed_element_kernel<Op, BWD>), dim3((unsigned)grid), dim3(kBlock), 0,
                            hs(stream), grad_out, packed, out, rows, h);
         return hipGetLastError();
     }
-    const uint32_t hv = (uint32_t)(h / 8);
-    const FastDiv div = make_fastdiv(hv);
+    const PackedShape sh{(uint32_t)n_vec, (uint32_t)nv, (uint32_t)h, make_fastdiv((uint32_t)nv)};
     const int64_t grid = grid_one_pass(n_vec);
     // bytes: forward reads gate+up (4n) and writes 2n; backward reads
     // grad_out+gate+up (6n) and writes 4n.
@@ -129,10 +168,10 @@ int launch_packed(void* out, const void* grad_out, const void* packed, int64_t r
 #define PT_PACKED_LAUNCH(LNT, SNT)                                                              \
     if constexpr (BWD)                                                                         \
         hipLaunchKernelGGL((packed_bwd_kernel<Op, LNT, SNT>), dim3((unsigned)grid), dim3(kBlock), \
-                           0, hs(stream), grad_out, packed, out, (uint32_t)n_vec, hv, div);     \
+                           0, hs(stream), grad_out, packed, out, sh);                           \
     else                                                                                       \
         hipLaunchKernelGGL((packed_fwd_kernel<Op, LNT, SNT>), dim3((unsigned)grid), dim3(kBlock), \
-                           0, hs(stream), packed, out, (uint32_t)n_vec, hv, div);
+                           0, hs(stream), packed, out, sh);
     if (mode == kNtBoth) {
         PT_PACKED_LAUNCH(true, true)
     } else if (mode == kNtStore) {

@@ -148,6 +148,40 @@ def test_packed_matches_separate(capi, cuda, degree, fmt, hidden):
         assert torch.equal(grad_p.view(torch.int16), torch.cat((gg, gu), -1).view(torch.int16))
 
 
+@pytest.mark.parametrize("rows,hidden,offset", [
+    (1, 8, 0), (5, 8, 2), (5, 14, 0), (5, 14, 1), (3, 15, 0), (3, 4, 2), (257, 1366, 2), (65, 2730, 0),
+    (17000, 2730, 0)])  # the last one loads and stores non-temporally
+def test_packed_rows_of_any_width(capi, cuda, rows, hidden, offset):
+    """Row vectors that overlap at a row's end (H no multiple of 8), storage
+    that starts `offset` elements into an allocation: equal to the separate
+    kernels bit for bit, and nothing outside the outputs is written."""
+    torch.manual_seed(hidden + offset)
+    n, guard = rows * hidden, 64
+
+    def buffer(count, value=None):
+        t = torch.full((count + offset + 2 * guard,), 7.0, device=cuda, dtype=torch.bfloat16)
+        view = t[guard + offset:guard + offset + count]
+        if value is not None:
+            view.copy_(value.reshape(-1))
+        return t, view
+
+    values = (torch.randn(rows, 2 * hidden, device=cuda) * 3).to(torch.bfloat16)
+    grads = torch.randn(rows, hidden, device=cuda).to(torch.bfloat16)
+    gate, up = (p.contiguous() for p in values.chunk(2, dim=-1))
+    (_, packed), (_, go) = buffer(2 * n, values), buffer(n, grads)
+    (out_all, out), (grad_all, grad) = buffer(n), buffer(2 * n)
+    capi.call("launch_swish_mul_packed_fwd_d3_kernel_bf16", out, packed, rows, hidden)
+    capi.call("launch_swish_mul_packed_bwd_d3_kernel_bf16", grad, go, packed, rows, hidden)
+    want, gg, gu = torch.empty_like(gate), torch.empty_like(gate), torch.empty_like(gate)
+    capi.call("launch_swish_mul_fwd_d3_kernel_bf16", want, gate, up, n)
+    capi.call("launch_swish_mul_bwd_d3_kernel_bf16", gg, gu, grads, gate, up, n)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16).reshape(-1))
+    assert torch.equal(grad.view(torch.int16), torch.cat((gg, gu), -1).view(torch.int16).reshape(-1))
+    for whole, count in ((out_all, n), (grad_all, 2 * n)):
+        assert bool((whole[:guard + offset] == 7).all()) and bool((whole[guard + offset + count:] == 7).all())
+
+
 def test_b3_exhaustive(capi, oracle, cuda):
     x = oracle.all_bits()
     xd = _dev(x, "bf16", cuda)
