@@ -18,11 +18,11 @@
 // s = q.k * scale.
 //
 // Design (all-transposed MFMA formulation, v_mfma_f32_32x32x16_bf16):
-//  * a block of 4 or 8 waves owns 128 or 256 queries (launch_fwd picks by
-//    head_dim and mode); each wave owns 32 queries, held
-//    as the B operand Q^T (8 fragments of 8 BF16 per lane, loaded once);
-//  * the block stages 64-key tiles of K and V in LDS, both row-major as they
-//    arrive (16-byte stores, padded rows);
+//  * a block of 4 or 8 waves owns 32 queries per wave, held as the B operand
+//    Q^T (fragments of 8 BF16 per lane);
+//  * 64-key tiles of K and V move from memory straight into rings of LDS
+//    tiles (load_to_lds, swizzled rows), two tiles ahead at head_dim 128; Q
+//    takes the same way once, through the V ring;
 //  * S^T = K Q^T: lane (h, c) of a wave accumulates 16 keys x query c for
 //    each 32-key tile, so every per-query reduction is lane-local plus one
 //    exchange with lane c + 32;
@@ -32,14 +32,21 @@
 //    tile in the same order through gfx950's transposing LDS reads
 //    (ds_read_b64_tr_b16, two per fragment), and O^T keeps each lane on its
 //    own query, so the online-softmax rescale is lane-local too;
-//  * the next K / V tile is loaded into registers while the current one is
-//    used and written to the second LDS buffer afterwards (one barrier per
-//    tile);
+//  * one barrier per tile.  With 8 waves, two to a SIMD, waves 0-3 meet it
+//    ahead of S and waves 4-7 ahead of O += P V, so the two waves of a SIMD
+//    stay half a tile apart and one's MFMAs meet the other's score program;
+//  * O leaves through LDS, whole rows to memory;
 //  * causal blocks run from the heaviest query block down.
+//
+// What bounds it: the score program's issue slots next to the matrix cores
+// (head_dim 128, causal, S 4096, 32 query heads: the MFMAs alone take 63 us of
+// the SIMDs), and the power budget: the clock is 2.05 GHz here and 1.8 GHz
+// where MFMAs run back to back.
 #include <hip/hip_runtime.h>
 
 #include "flash_attn.hpp"
 #include "spline_ops_hip.h"
+
 
 namespace pt {
 
@@ -58,7 +65,30 @@ struct AttnParams {
     int causal;
     int route;       // exp2 route of the kRouteRuntime instantiations
     uint32_t rmask;  // and its periodic mask (routes up to 32)
+    int group;       // query heads per KV head
+    int wide;        // a row stride too large for 32-bit lane offsets
 };
+
+// Launch constants of the score programs, in VGPRs (vgpr()).
+struct ScoreConsts {
+    float scale;    // s = q.k * scale
+    float sl;       // softmax modes: log2 e times the unit of the exponents
+    float cap, inv_cap, bias;
+    float tanh[SoftcapConsts::T::P.deg + 1];  // softcap D4
+};
+
+template <int MODE>
+__device__ __forceinline__ ScoreConsts score_consts(const AttnParams& p) {
+    ScoreConsts c;
+    c.scale = vgpr(p.scale);
+    c.sl = vgpr(attn_is_plain_softmax(MODE) ? p.scale * kLog2e : kLog2e);
+    c.cap = vgpr(p.cap);
+    c.inv_cap = vgpr(1.0f / p.cap);
+    c.bias = vgpr(p.sig_bias);
+#pragma unroll
+    for (int i = 1; i <= SoftcapConsts::T::P.deg; ++i) c.tanh[i] = vgpr(bf16_value(SoftcapConsts::T::P.c[i]));
+    return c;
+}
 
 // Softmax scores of 16 accumulator registers (one 32-key tile), in the
 // units the caller's exponent FMA scales by sl: the raw dot products for
@@ -67,25 +97,21 @@ struct AttnParams {
 // The D4 program runs on BF16 pairs: u = bf16(bf16(s) * (1/cap)),
 // y = bf16(cap * TANH_D4_BF16(u)), the B2 program on the BF16 score.
 template <int MODE>
-__device__ __forceinline__ void softmax_exponents(const f32x16_t& acc, float scale, float cap,
-                                                  float inv_cap, float (&x)[16]) {
+__device__ __forceinline__ void softmax_exponents(const f32x16_t& acc, const ScoreConsts& k, float (&x)[16]) {
     if constexpr (MODE == kAttnSoftcapD4) {
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {
-            const uint32_t u = pack_bf(rbf(acc[r] * scale) * inv_cap, rbf(acc[r + 1] * scale) * inv_cap);
+            const uint32_t u = pack_bf(rbf(acc[r] * k.scale) * k.inv_cap, rbf(acc[r + 1] * k.scale) * k.inv_cap);
             float t0, t1;
-            SoftcapConsts::T::eval2(u, t0, t1);
-            x[r] = rbf(t0 * cap);
-            x[r + 1] = rbf(t1 * cap);
+            SoftcapConsts::T::eval2(u, k.tanh, t0, t1);
+            x[r] = rbf(t0 * k.cap);
+            x[r + 1] = rbf(t1 * k.cap);
         }
-    } else if constexpr (MODE == kAttnSoftcapNative) {
+    } else {
+        static_assert(MODE == kAttnSoftcapNative, "plain softmax keeps the raw dot products");
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-            x[r] = cap * native_lane<kTanh, kFwd>(acc[r] * scale * inv_cap);
-    } else {
-        const float sl = scale * kLog2e;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = acc[r] * sl;
+            x[r] = k.cap * native_lane<kTanh, kFwd>(acc[r] * k.scale * k.inv_cap);
     }
 }
 
@@ -130,8 +156,8 @@ template <int MODE>
 __device__ __forceinline__ void sigmoid_prob2(float s0, float s1, float bias, float& p0, float& p1) {
     if constexpr (MODE == kAttnSigmoidB3) {
         float dy;
-        b3_lane<false, true>(rbf(s0), p0, dy);
-        b3_lane<false, true>(rbf(s1), p1, dy);
+        b3_lane<false, true, true>(rbf(s0), p0, dy);
+        b3_lane<false, true, true>(rbf(s1), p1, dy);
     } else if constexpr (MODE == kAttnSigmoidB3D2) {
         float dy;
         b3_d2_lane(rbf(s0), p0, dy);
@@ -150,13 +176,6 @@ __device__ __forceinline__ void sigmoid_prob2(float s0, float s1, float bias, fl
 // unchanged.  Most tiles skip the 64-register rescale of O.
 constexpr float kRescaleThreshold = 8.0f;
 
-// Modes whose score program dominates a tile's issue cycles: softcap D4 and
-// the sigmoid polynomials.
-template <int MODE>
-constexpr bool fwd_program_heavy() {
-    return MODE == kAttnSoftcapD4 || (attn_is_sigmoid(MODE) && MODE != kAttnSigmoidNative);
-}
-
 // Accumulator register r of 32-key tile kt holds key k0 + kt*32 + 8*(r/4) +
 // 4h + r%4; diag = k0 + 4h - klast, with klast the last key the query may
 // see (itself under the causal mask, at most the last real key), so the key
@@ -166,38 +185,14 @@ __device__ __forceinline__ bool key_masked(int diag, int kt, int r) {
     return MASKED && diag + kt * 32 + 8 * (r >> 2) + (r & 3) > 0;
 }
 
-// S^T = K Q^T for one 64-key tile (two 32-key accumulators, independent
-// chains interleaved).  PRIO: raised wave priority while this wave only
-// issues MFMA, so the other waves of the SIMD keep the VALU busy meanwhile
-// (measured on MI355X: 1-2 % faster for the light score programs, 1-4.5 %
-// slower for the heavy ones, whose VALU work should not wait).
-template <int HD, bool PRIO>
-__device__ __forceinline__ void tile_scores(const uint16_t* __restrict__ ks, const bf16x8_t (&qf)[HD / 16],
-                                            f32x16_t (&sacc)[2], int h, int c32) {
-    constexpr int kKStr = HD + 8;  // BF16 elements per LDS K row
-    sacc[0] = (f32x16_t){};
-    sacc[1] = (f32x16_t){};
-    if constexpr (PRIO) __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int c = 0; c < HD / 16; ++c)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-            const bf16x8_t a =
-                *reinterpret_cast<const bf16x8_t*>(ks + (kt * 32 + c32) * kKStr + c * 16 + h * 8);
-            sacc[kt] = mfma32(a, qf[c], sacc[kt]);
-        }
-    if constexpr (PRIO) __builtin_amdgcn_s_setprio(0);
-}
-
 // Softmax modes: exponents x of the tile (plain softmax keeps the raw dot
 // products and folds the scale into the exp2 argument, sl; softcap modes
 // transform first), masked keys to -inf, and the lazy online-max update,
 // which rescales O and l when this tile raises the maximum by more than the
 // threshold.  Sigmoid modes have no state to update.
 template <int MODE, bool MASKED, int HD>
-__device__ __forceinline__ void tile_softmax_state(const AttnParams& p, const f32x16_t (&sacc)[2], float (&x)[2][16],
-                                                   f32x16_t (&oacc)[HD / 32], float& m, float& l, int diag,
-                                                   float inv_cap, float sl) {
+__device__ __forceinline__ void tile_softmax_state(const ScoreConsts& k, const f32x16_t (&sacc)[2], float (&x)[2][16],
+                                                   f32x16_t (&oacc)[HD / 32], float& m, float& l, int diag) {
     if constexpr (!attn_is_sigmoid(MODE)) {
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -205,7 +200,7 @@ __device__ __forceinline__ void tile_softmax_state(const AttnParams& p, const f3
 #pragma unroll
                 for (int r = 0; r < 16; ++r) x[kt][r] = sacc[kt][r];
             } else {
-                softmax_exponents<MODE>(sacc[kt], p.scale, p.cap, inv_cap, x[kt]);
+                softmax_exponents<MODE>(sacc[kt], k, x[kt]);
             }
         }
         // max over four independent chains
@@ -217,14 +212,13 @@ __device__ __forceinline__ void tile_softmax_state(const AttnParams& p, const f3
                 if (key_masked<MASKED>(diag, kt, r)) x[kt][r] = -__builtin_inff();
                 mx[r & 3] = __builtin_fmaxf(mx[r & 3], x[kt][r]);
             }
-        float mt = __builtin_fmaxf(__builtin_fmaxf(mx[0], mx[1]), __builtin_fmaxf(mx[2], mx[3]));
-        mt = __builtin_fmaxf(mt, __shfl_xor(mt, 32)) * sl;
+        const float mt =
+            half_max(__builtin_fmaxf(__builtin_fmaxf(mx[0], mx[1]), __builtin_fmaxf(mx[2], mx[3]))) * k.sl;
         // lanes c and c + 32 hold the same query and take the same decision
         const bool move = mt > m + kRescaleThreshold;
         // scheduling fences around the rare rescale: without them the
         // scheduler interleaves it with the surrounding code and the register
         // allocator then copies all of O on the common no-rescale path
-        // (head_dim 64: 34 moves per tile)
         __builtin_amdgcn_sched_barrier(0);
         if (__any(move)) {
             const float m_use = move ? mt : m;
@@ -242,15 +236,15 @@ __device__ __forceinline__ void tile_softmax_state(const AttnParams& p, const f3
 // layout) as the BF16 B operand of one O^T MFMA; softmax modes add them to
 // the four row-sum chains ls.
 template <int MODE, int ROUTE, bool MASKED>
-__device__ __forceinline__ bf16x8_t tile_probs8(const AttnParams& p, const f32x16_t (&sacc)[2],
-                                                const float (&x)[2][16], int kt, int cc, float sl, float m,
-                                                int diag, uint32_t rmask, float (&ls)[4]) {
+__device__ __forceinline__ bf16x8_t tile_probs8(const ScoreConsts& k, const f32x16_t (&sacc)[2],
+                                                const float (&x)[2][16], int kt, int cc, float m, int diag,
+                                                uint32_t rmask, float (&ls)[4]) {
     float pr[8];
     if constexpr (attn_is_sigmoid(MODE)) {
 #pragma unroll
         for (int e = 0; e < 8; e += 2) {
             const int r = 8 * cc + e;
-            sigmoid_prob2<MODE>(sacc[kt][r] * p.scale, sacc[kt][r + 1] * p.scale, p.sig_bias, pr[e], pr[e + 1]);
+            sigmoid_prob2<MODE>(sacc[kt][r] * k.scale, sacc[kt][r + 1] * k.scale, k.bias, pr[e], pr[e + 1]);
             pr[e] = key_masked<MASKED>(diag, kt, r) ? 0.0f : pr[e];
             pr[e + 1] = key_masked<MASKED>(diag, kt, r + 1) ? 0.0f : pr[e + 1];
         }
@@ -259,7 +253,7 @@ __device__ __forceinline__ bf16x8_t tile_probs8(const AttnParams& p, const f32x1
         for (int e = 0; e < 8; e += 2) {
             const int r = 8 * cc + e;
             float ev0, ev1;
-            softmax_exp2_pair<MODE, ROUTE>(__builtin_fmaf(x[kt][r], sl, -m), __builtin_fmaf(x[kt][r + 1], sl, -m),
+            softmax_exp2_pair<MODE, ROUTE>(__builtin_fmaf(x[kt][r], k.sl, -m), __builtin_fmaf(x[kt][r + 1], k.sl, -m),
                                            kt * 16 + r, rmask, ev0, ev1);
             pr[e] = key_masked<MASKED>(diag, kt, r) ? 0.0f : ev0;
             pr[e + 1] = key_masked<MASKED>(diag, kt, r + 1) ? 0.0f : ev1;
@@ -270,7 +264,7 @@ __device__ __forceinline__ bf16x8_t tile_probs8(const AttnParams& p, const f32x1
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int r = 8 * cc + e;
-            const float ev = softmax_exp2<MODE, ROUTE>(__builtin_fmaf(x[kt][r], sl, -m), kt * 16 + r, rmask);
+            const float ev = softmax_exp2<MODE, ROUTE>(__builtin_fmaf(x[kt][r], k.sl, -m), kt * 16 + r, rmask);
             // v_exp_f32(-inf) is 0; the polynomial programs clamp at -127
             pr[e] = (attn_has_exp2_program(MODE) && key_masked<MASKED>(diag, kt, r)) ? 0.0f : ev;
             ls[e & 3] += pr[e];
@@ -282,211 +276,256 @@ __device__ __forceinline__ bf16x8_t tile_probs8(const AttnParams& p, const f32x1
     return pf;
 }
 
-// O^T += V^T P^T for the eight keys of tile_probs8(kt, cc): the V^T fragment
-// of dims dt*32 + (lane % 32), keys kt*32 + cc*16 + 4h + {0..3, 8..11} comes
-// from two transposing reads of the row-major V tile (vrow points at this
-// lane's source chunk of the first).
-template <int HD>
-__device__ __forceinline__ void tile_pv8(const uint16_t* __restrict__ vrow, int kt, int cc, bf16x8_t pf,
-                                         f32x16_t (&oacc)[HD / 32]) {
-#pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt) {
-        const uint16_t* src = vrow + (kt * 32 + cc * 16) * kVRowStr<HD>() + dt * 32;
-        const v4i16_t lo = lds_read_tr16(src);
-        const v4i16_t hi = lds_read_tr16(src + 8 * kVRowStr<HD>());
-        const u32x4_t w = {__builtin_bit_cast(u32x2_t, lo).x, __builtin_bit_cast(u32x2_t, lo).y,
-                           __builtin_bit_cast(u32x2_t, hi).x, __builtin_bit_cast(u32x2_t, hi).y};
-        oacc[dt] = mfma32(__builtin_bit_cast(bf16x8_t, w), pf, oacc[dt]);
-    }
-}
+// Shape of the forward: waves (32 queries each) per block and tiles per LDS
+// ring.  head_dim 128: 8 waves that share each staged tile, one block per CU
+// with four tiles of K and of V in 130 KiB, or two independent 4-wave blocks
+// with two tiles each (fwd_waves picks); head_dim 64: three independent
+// 4-wave blocks per CU, three tiles each in 50 KiB.
+template <int HD, int W>
+struct FwdShape {
+    static constexpr int kWaves = W;
+    static constexpr int kRing = HD == 64 ? 3 : W == 8 ? 4 : 2;
+    static constexpr int kBlockQ = 32 * kWaves;
+    static constexpr int kRowB = HD * 2;                      // bytes per row
+    static constexpr int kTileB = lds_row<HD>(kAttnBlockK);  // bytes per staged tile
+    static constexpr int kChunks = RowLoader<HD>::kChunks, kLoadRows = RowLoader<HD>::kLoadRows;
+    static constexpr int kLoads = kAttnBlockK / kLoadRows / kWaves;  // per wave, tile and operand
+    static_assert(lds_row<HD>(kBlockQ) <= kRing * kTileB, "Q passes through the V ring");
+};
 
-// One 64-key tile for one wave: S^T = K Q^T, the score program, the online
-// softmax (or sigmoid) and O^T += V^T P^T.  MASKED: the tile crosses the
-// causal diagonal of this wave's 32 queries.  Probabilities are produced
-// eight at a time right before the O^T MFMAs that consume them, so the
-// exponentials of one group issue while the previous group's MFMAs run.
-template <int MODE, int ROUTE, bool MASKED, int HD>
-__device__ __forceinline__ void attend_tile(const AttnParams& p, const uint16_t* __restrict__ ks,
-                                            const uint16_t* __restrict__ vrow, const bf16x8_t (&qf)[HD / 16],
-                                            f32x16_t (&oacc)[HD / 32], float& m, float& l, int diag,
-                                            int h, int c32, float inv_cap, uint32_t rmask) {
-    f32x16_t sacc[2];
-    tile_scores<HD, !fwd_program_heavy<MODE>()>(ks, qf, sacc, h, c32);
-    float x[2][16];
-    float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    const float sl = attn_is_plain_softmax(MODE) ? p.scale * kLog2e : kLog2e;
-    tile_softmax_state<MODE, MASKED, HD>(p, sacc, x, oacc, m, l, diag, inv_cap, sl);
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int cc = 0; cc < 2; ++cc)
-            tile_pv8<HD>(vrow, kt, cc, tile_probs8<MODE, ROUTE, MASKED>(p, sacc, x, kt, cc, sl, m, diag, rmask, ls), oacc);
-    if constexpr (!attn_is_sigmoid(MODE)) l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+// Waves per SIMD the register allocation is held to: 2 at head_dim 128 (256
+// VGPRs); the head_dim-64 kernels fit three 4-wave blocks per CU (168 VGPRs)
+// except the softcap modes (172 and 175).
+template <int MODE, int HD>
+constexpr int fwd_waves_per_eu() {
+    return HD == 64 && MODE != kAttnSoftcapD4 && MODE != kAttnSoftcapNative ? 3 : 2;
 }
 
 // Grid (q_heads, ceil(S / (32 W)), batch), W waves of 32 queries per block:
 // blockIdx.y runs over query blocks, heaviest first under the causal mask,
 // and the head index varies fastest, so the first wave of resident blocks
 // takes the longest query blocks of every head.
-// RAGGED: S is not a multiple of 128, so the last query block and the last
-// key tile hold rows past the sequence, or keys from kv_len on are padding
-// (a separate instantiation keeps those guards out of the aligned kernels).
-// Waves per SIMD the register allocation is held to: 2 (up to 256 VGPRs).
-// The head_dim-64 kernels fit three 4-wave blocks per CU (<= 168 VGPRs)
-// by themselves, except the packed FP16 exp2 programs, whose packed pairs
-// keep more values live (170 VGPRs for the PWL2 hinge at route 12): they are
-// held to 3 where that costs no spill (routes above 8; at 4 and 8 the hinge
-// would spill 2-17 registers).
-template <int MODE, int ROUTE, int HD>
-constexpr int fwd_waves_per_eu() {
-    return HD == 64 && exp2_is_f16(attn_exp2_kind<MODE>()) && ROUTE > 8 ? 3 : 2;
-}
-
-template <int MODE, int ROUTE, int HD, int W, bool RAGGED>
+//
+// Any S: rows past the last real key are staged as that key's row (a finite
+// row times a masked probability, which is 0), queries past the sequence
+// compute the last query's row and store nothing, and a wave with no query
+// at all only stages.
+template <int MODE, int ROUTE, int HD, int W>
 __global__ void __launch_bounds__(64 * W)
-    __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu<MODE, ROUTE, HD>()))) flash_fwd_kernel(AttnParams p) {
-    constexpr int kBlockQ = 32 * W;  // queries per block
+    __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu<MODE, HD>()))) flash_fwd_kernel(AttnParams p) {
+    using F = FwdShape<HD, W>;
+    constexpr int kRing = F::kRing, kRowB = F::kRowB, kTileB = F::kTileB;
     constexpr bool kSigmoid = attn_is_sigmoid(MODE);
-    constexpr int kKStr = HD + 8;
-    // two buffers: the next tile is written while the current one is read;
-    // K and V are both row-major (V^T fragments come from transposing reads)
-    __shared__ __align__(16) uint16_t ks[2][kAttnBlockK * kKStr];
-    __shared__ __align__(16) uint16_t vs[2][kAttnBlockK * kVRowStr<HD>()];
+    constexpr bool kLate = W == 8;  // the second wave of each SIMD runs half a tile behind
+    constexpr int kAheadV = kLate ? kRing - 2 : kRing - 1, kInFlight = kLate ? kRing - 3 : kRing - 2;
+    constexpr int kC = HD / 16, kD = HD / 32;
+    // K ring, V ring
+    __shared__ __align__(1024) unsigned char smem[2 * kRing * kTileB];
+    constexpr uint32_t kV = kRing * kTileB;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int h = lane >> 5, c32 = lane & 31;
-    const int64_t nqb = (p.seq + kBlockQ - 1) / kBlockQ;  // the last block may be partial
-    const int64_t head = blockIdx.x, b = blockIdx.z;
-    const int64_t qb = p.causal ? nqb - 1 - (int64_t)blockIdx.y : (int64_t)blockIdx.y;
-    const int64_t kvh = head / (p.hq / p.hkv);
+    const int seq = (int)p.seq, klim = (int)p.kv_len - 1;  // the last real key
+    const int nqb = (seq + F::kBlockQ - 1) / F::kBlockQ;
+    const int head = blockIdx.x, b = blockIdx.z;
+    const int qb = p.causal ? nqb - 1 - (int)blockIdx.y : (int)blockIdx.y;
+    const int kvh = (int)((uint32_t)head / (uint32_t)p.group);
     const uint16_t* qp = p.q + b * p.qs.b + head * p.qs.h;
     const uint16_t* kp = p.k + b * p.ks.b + kvh * p.ks.h;
     const uint16_t* vp = p.v + b * p.vs.b + kvh * p.vs.h;
-    const int64_t kss = p.ks.s, vss = p.vs.s;
-    const int64_t q0 = qb * kBlockQ + wave * 32;  // first query of this wave
-    const int64_t qrow = q0 + c32;                     // this lane's query
+    const int q0 = qb * F::kBlockQ + wave * 32;  // first query of this wave
+    const int qrow = q0 + c32;                   // this lane's query
+    const bool qin = qrow < seq;
 
-    // queries past the sequence (the last block of a length that is not a
-    // multiple of the block) load the last row and are zeroed before the
-    // tile loop; their outputs are not stored.  The loads stay unconditional:
-    // a branch around each would wait for every load before the next.
-    const bool qin = !RAGGED || qrow < p.seq;
-    const int64_t qsrc = qin ? qrow : p.seq - 1;
-    bf16x8_t qf[HD / 16];
-#pragma unroll
-    for (int c = 0; c < HD / 16; ++c)
-        qf[c] = *reinterpret_cast<const bf16x8_t*>(qp + qsrc * p.qs.s + c * 16 + h * 8);
+    // the last visible key of this lane's query, and of the wave's queries
+    const int klast = p.causal && qrow < klim ? qrow : klim;
+    const int whi = p.causal && q0 + 31 < klim ? q0 + 31 : klim;
+    // key tiles of the block and of this wave (none without a query)
+    const int ktiles = klim / kAttnBlockK + 1;
+    const int ncausal = p.causal ? (qb + 1) * (F::kBlockQ / kAttnBlockK) : ktiles;
+    const int nkb = ncausal < ktiles ? ncausal : ktiles;
+    const int nw = q0 < seq ? whi / kAttnBlockK + 1 : 0;
 
-    f32x16_t oacc[HD / 32];
+    // ---- staging: load j of a wave moves rows kLoadRows (W j + wave) ..
+    const RowLoader<HD> loader(lane, p.wide);
+    const TileReader<HD> reader(lane);
+    auto load_tile = [&](uint32_t lds, const uint16_t* base, int64_t stride, int t) {
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt) oacc[dt] = (f32x16_t){};
+        for (int j = 0; j < F::kLoads; ++j) {
+            const int r = F::kLoadRows * (j * W + wave);
+            loader.load(lds + lds_row<HD>(r), F::kLoadRows * wave, base, stride, t * kAttnBlockK + r, klim);
+        }
+    };
+    auto load_k = [&](int t) { load_tile(lds0 + (uint32_t)(t % kRing * kTileB), kp, p.ks.s, t); };
+    auto load_v = [&](int t) { load_tile(lds0 + kV + (uint32_t)(t % kRing * kTileB), vp, p.vs.s, t); };
+
+    // ---- prologue: K(0), Q through the V ring, the K tiles ahead
+    load_k(0);
+#pragma unroll
+    for (int j = 0; j < 32 / F::kLoadRows; ++j) {
+        const int r = F::kLoadRows * (j * W + wave);
+        loader.load(lds0 + kV + lds_row<HD>(r), F::kLoadRows * wave, qp, p.qs.s, qb * F::kBlockQ + r, seq - 1);
+    }
+#pragma unroll
+    for (int t = 1; t < kRing - 1; ++t)
+        if (t < nkb) load_k(t);
+
+    const ScoreConsts k = score_consts<MODE>(p);
+    f32x16_t oacc[kD];
+#pragma unroll
+    for (int dt = 0; dt < kD; ++dt) oacc[dt] = (f32x16_t){};
     float m = -__builtin_inff(), l = 0.0f;
-    const float inv_cap = 1.0f / p.cap;
 
-    // staging: K and V rows krow + kRowsPass j, 16 bytes at kcol
-    constexpr int kChunks = HD / 8;                   // 16-byte chunks per row
-    constexpr int kRowsPass = 64 * W / kChunks;       // rows per pass
-    constexpr int kPasses = kAttnBlockK / kRowsPass;
-    const int krow = tid / kChunks, kcol = (tid % kChunks) * 8;
-    u32x4_t kr[kPasses], vr[kPasses];
-    auto load = [&](int64_t k0) {
-        if (!RAGGED || k0 + kAttnBlockK <= p.seq) {  // block-uniform: a whole tile of rows
+    wait_loads<0>();
+    block_barrier();
+    bf16x8_t qf[kC];
 #pragma unroll
-            for (int j = 0; j < kPasses; ++j) {
-                kr[j] = *reinterpret_cast<const u32x4_t*>(kp + (k0 + krow + kRowsPass * j) * kss + kcol);
-                vr[j] = *reinterpret_cast<const u32x4_t*>(vp + (k0 + krow + kRowsPass * j) * vss + kcol);
-            }
-        } else {  // the sequence ends inside the tile: rows past it read the
-                  // last row (unconditional loads) and are zeroed by the store
+    for (int c = 0; c < kC; ++c) qf[c] = reader.row_frag(smem + kV + lds_row<HD>(wave * 32), c);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    block_barrier();  // every wave has its Q fragments: the V ring is free
 #pragma unroll
-            for (int j = 0; j < kPasses; ++j) {
-                const int64_t row = k0 + krow + kRowsPass * j;
-                const int64_t src = row < p.seq ? row : p.seq - 1;
-                kr[j] = *reinterpret_cast<const u32x4_t*>(kp + src * kss + kcol);
-                vr[j] = *reinterpret_cast<const u32x4_t*>(vp + src * vss + kcol);
+    for (int t = 0; t < kAheadV; ++t)
+        if (t < nkb) load_v(t);
+
+    // sync(i): K(i), V(i) and older tiles have landed for every wave, and every
+    // wave is done with tile i - 1, late waves but for its P V.  Loads K of
+    // kRing - 1 tiles ahead over K(i - 1), V as far ahead over V(i - 1), or one
+    // tile less over V(i - 2) where late waves still read V(i - 1).  The loads
+    // of kRing - 2 tiles (one less with late waves) may still be in flight.
+    auto sync = [&](int i) {
+        if (kInFlight > 0 && i > 0 && i + kInFlight + (kLate ? 1 : 0) < nkb) wait_loads<2 * F::kLoads * kInFlight>();
+        else wait_loads<0>();
+        block_barrier();
+        if (i + kRing - 1 < nkb) load_k(i + kRing - 1);
+        if (i + kAheadV < nkb) load_v(i + kAheadV);
+    };
+    // S^T = K Q^T of tile i: two 32-key accumulators, independent chains
+    // interleaved, six fragments read ahead where two waves run in step
+    f32x16_t s[2];
+    auto scores = [&](int i) {
+        const uint32_t tile = (uint32_t)(i % kRing * kTileB);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!kLate) __builtin_amdgcn_s_setprio(1);  // the other blocks keep the VALU busy meanwhile
+        s[0] = s[1] = (f32x16_t){};
+#pragma unroll
+        for (int c = 0; c < kC; ++c)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) s[kt] = mfma32(reader.row_frag(smem + tile + lds_row<HD>(kt * 32), c), qf[c], s[kt]);
+        if constexpr (kLate) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+            for (int g = 0; g < 2 * kC - 6; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             }
+            __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+        }
+        if constexpr (!kLate) __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // O^T += V^T P^T of the 16 keys g
+    bf16x8_t pf[4];
+    auto accumulate8 = [&](uint32_t tile, int g) {
+#pragma unroll
+        for (int dt = 0; dt < kD; ++dt)
+            oacc[dt] = mfma32(reader.col_frag(smem + tile + lds_row<HD>(16 * g), dt), pf[g], oacc[dt]);
+    };
+    // With independent 4-wave blocks the polynomial programs run faster with
+    // each 16 keys' products right behind their probabilities (head_dim 64,
+    // causal, S 4096, 32 heads: B3 143 against 150 us, D2 at 4 of 12 111
+    // against 114; hardware exp2 101 and softcap 202 against 103 and 208 the
+    // other way).
+    constexpr bool kFused = HD == 64 && (attn_has_exp2_program(MODE) || kSigmoid);
+    // probabilities of tile i (masked: it holds the causal diagonal of the
+    // wave's queries or keys past the last) as the B operands of P V
+    auto probabilities = [&](auto masked_c, int i) {
+        constexpr bool MASKED = decltype(masked_c)::value;
+        const int diag = i * kAttnBlockK - klast + 4 * h;
+        const uint32_t rmask = ROUTE == kRouteRuntime ? tile_route_mask(p.route, p.rmask, i) : 0u;
+        float x[2][16];
+        float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        tile_softmax_state<MODE, MASKED, HD>(k, s, x, oacc, m, l, diag);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            pf[g] = tile_probs8<MODE, ROUTE, MASKED>(k, s, x, g >> 1, g & 1, m, diag, rmask, ls);
+            if constexpr (kFused) accumulate8(kV + (uint32_t)(i % kRing * kTileB), g);
+        }
+        if constexpr (!kSigmoid) l += (ls[0] + ls[1]) + (ls[2] + ls[3]);
+    };
+    // the products of tile i, three fragments read ahead
+    auto accumulate = [&](int i) {
+        if constexpr (!kFused) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) accumulate8(kV + (uint32_t)(i % kRing * kTileB), g);
+            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+            for (int g = 0; g < 4 * kD - 3; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // rows from kv_len on (padding keys, and rows past the sequence) are
-    // zeroed before they reach LDS, so whatever the padding holds (NaN, Inf)
-    // the masked P (0) times V stays 0
-    auto store = [&](int buf, int64_t k0) {
-        if (RAGGED && k0 + kAttnBlockK > p.kv_len) {  // block-uniform: the tile holds rows from kv_len on
-#pragma unroll
-            for (int j = 0; j < kPasses; ++j)
-                if (k0 + krow + kRowsPass * j >= p.kv_len) kr[j] = vr[j] = (u32x4_t){0u, 0u, 0u, 0u};
-        }
-#pragma unroll
-        for (int j = 0; j < kPasses; ++j) {
-            *reinterpret_cast<u32x4_t*>(&ks[buf][(krow + kRowsPass * j) * kKStr + kcol]) = kr[j];
-            *reinterpret_cast<u32x4_t*>(&vs[buf][(krow + kRowsPass * j) * kVRowStr<HD>() + kcol]) = vr[j];
-        }
-    };
-    // this lane's source chunk of the transposing V reads: key (lane % 16) / 4
-    // + 4h, dims 16 ((lane / 16) % 2) + 4 (lane % 4) of a 32-dim slice
-    const int vlane = (((lane & 15) >> 2) + 4 * h) * kVRowStr<HD>() + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 
-    // the last visible key of this lane's query and the smallest and largest
-    // of those over the wave's 32 queries (wave-uniform)
-    const int64_t klim = p.kv_len - 1;
-    const int64_t klast = p.causal && qrow < klim ? qrow : klim;
-    const int64_t wlo = p.causal && q0 < klim ? q0 : klim;
-    const int64_t whi = p.causal && q0 + 31 < klim ? q0 + 31 : klim;
-    const int64_t ktiles = (p.kv_len + kAttnBlockK - 1) / kAttnBlockK;  // tiles holding real keys
-    const int64_t ncausal = p.causal ? (qb + 1) * (kBlockQ / kAttnBlockK) : ktiles;
-    const int64_t nkb = ncausal < ktiles ? ncausal : ktiles;
-    load(0);
-    store(0, 0);
-    // every load issued so far (the Q fragments included) completes before
-    // the loop: otherwise the counter waits the compiler places for the Q
-    // fragments inside the loop also wait for the next tile's prefetch
-    __builtin_amdgcn_s_waitcnt(0);
-    if (!qin) {
-#pragma unroll
-        for (int c = 0; c < HD / 16; ++c) qf[c] = __builtin_bit_cast(bf16x8_t, (u32x4_t){0u, 0u, 0u, 0u});
+    // Late waves (the second wave of each SIMD) meet sync(i + 1) between the
+    // score program and P V of tile i, the others ahead of S(i + 1).
+    const bool late = kLate && wave >= 4;
+    sync(0);
+    int i = 0;
+    for (; i + 1 < nw; ++i) {
+        scores(i);
+        probabilities(std::integral_constant<bool, false>{}, i);
+        if (late) sync(i + 1);
+        accumulate(i);
+        if (!late) sync(i + 1);
     }
-    __syncthreads();
-    for (int64_t kb = 0; kb < nkb; ++kb) {
-        const int buf = (int)(kb & 1);
-        const int64_t k0 = kb * kAttnBlockK;
-        const bool more = kb + 1 < nkb;
-        if (more) load(k0 + kAttnBlockK);  // in flight during this tile's math
-        if (k0 <= whi) {  // wave-uniform: some key of the tile is visible
-            const int diag = (int)(k0 - klast) + 4 * h;
-            const uint32_t rmask = ROUTE == kRouteRuntime ? tile_route_mask(p.route, p.rmask, (int)kb) : 0u;
-            if (k0 + kAttnBlockK - 1 > wlo)
-                attend_tile<MODE, ROUTE, true, HD>(p, ks[buf], vs[buf] + vlane, qf, oacc, m, l, diag, h, c32, inv_cap,
-                                                   rmask);
-            else
-                attend_tile<MODE, ROUTE, false, HD>(p, ks[buf], vs[buf] + vlane, qf, oacc, m, l, diag, h, c32, inv_cap,
-                                                    rmask);
-        }
-        if (more) store(buf ^ 1, k0 + kAttnBlockK);
-        __syncthreads();
+    int synced = i;  // sync(0) .. sync(synced) met
+    if (nw > 0) {  // the wave's last tile
+        scores(i);
+        probabilities(std::integral_constant<bool, true>{}, i);
+        if (late && i + 1 < nkb) sync(++synced);
+        accumulate(i);
     }
+    while (synced + 1 < nkb) sync(++synced);
+    if (nw == 0) return;
 
-    // ---- normalise and store: oacc[dt][r] = O^T[dt*32 + 8*(r/4) + 4h + r%4][qrow] ----
+    // ---- normalise and store: oacc[dt][r] = O^T[dt*32 + 8*(r/4) + 4h + r%4][qrow]
+    // through LDS, so that whole rows reach memory.  After sync(nkb - 1) the
+    // other waves read K(nkb - 1), V(nkb - 1) and V(nkb - 2) only: wave w
+    // takes part w % 2 of free K tile w / 2, the last two waves a free V tile.
     float inv = 1.0f;
     if constexpr (!kSigmoid) {
-        l += __shfl_xor(l, 32);
+        l = half_sum(l);
         inv = 1.0f / l;
         // log sum exp(s') with s' the (capped) scaled score: m and log2(l) are
         // in log2 units
         if (p.lse != nullptr && h == 0 && qin)
-            p.lse[(b * p.hq + head) * p.seq + qrow] = (m + __builtin_log2f(l)) * kLn2;
+            p.lse[((int64_t)b * p.hq + head) * seq + qrow] = (m + __builtin_log2f(l)) * kLn2;
     }
-    if (!qin) return;
-    uint16_t* orow = p.o + b * p.os.b + head * p.os.h + qrow * p.os.s;
+    const int part = wave >> 1;  // 32 rows are half a tile
+    const uint32_t slot = part < kRing - 1 ? (uint32_t)((nkb + part) % kRing * kTileB)
+                                           : kV + (uint32_t)(nkb % kRing * kTileB);
+    unsigned char* orows = smem + slot + (wave & 1) * 32 * kRowB;
 #pragma unroll
-    for (int dt = 0; dt < HD / 32; ++dt)
+    for (int dt = 0; dt < kD; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int d = dt * 32 + 8 * g + 4 * h;
-            const u32x2_t w = {pack_bf(oacc[dt][4 * g] * inv, oacc[dt][4 * g + 1] * inv),
-                               pack_bf(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv)};
-            *reinterpret_cast<u32x2_t*>(orow + d) = w;
-        }
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<u32x2_t*>(orows + c32 * kRowB + ((dt * 4 + g) ^ (c32 & (F::kChunks - 1))) * 16 + h * 8) =
+                (u32x2_t){pack_bf(oacc[dt][4 * g] * inv, oacc[dt][4 * g + 1] * inv),
+                          pack_bf(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv)};
+    __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
+    uint16_t* op = p.o + b * p.os.b + head * p.os.h;
+#pragma unroll
+    for (int j = 0; j < 32 / F::kLoadRows; ++j) {
+        const int r = j * F::kLoadRows + loader.lr;
+        const u32x4_t w =
+            *reinterpret_cast<const u32x4_t*>(orows + r * kRowB + (loader.lc ^ (r & (F::kChunks - 1))) * 16);
+        if (q0 + r < seq) *reinterpret_cast<u32x4_t*>(op + (q0 + r) * p.os.s + loader.lc * 8) = w;
+    }
 }
 
 }  // namespace pt
@@ -499,54 +538,47 @@ namespace {
 // the ones without a template instantiation take kRouteRuntime
 bool route_supported(int route) { return route >= 4 && route % 2 == 0; }
 
-// Waves (32 queries each) per block.  head_dim 128 runs 8-wave blocks (each
-// staged K / V tile serves 256 queries; one block per CU) except the modes
-// whose score program dominates the tile (softcap D4, the sigmoid polynomials),
-// which keep two independent 4-wave blocks per CU; head_dim 64 fits three
-// 4-wave blocks per CU and keeps them (measured on MI355X: 1.03-1.11x for the
-// softmax and hardware modes at D 128, 0.81-0.96x for 8 waves at D 64).
 template <int MODE, int ROUTE, int HD, int W>
-void launch_fwd_shape(const AttnParams& prm, dim3 grid, hipStream_t st) {
-    if (prm.seq % kAttnBlockQ == 0 && prm.kv_len == prm.seq)
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, HD, W, false>), grid, dim3(64 * W), 0, st, prm);
-    else
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, HD, W, true>), grid, dim3(64 * W), 0, st, prm);
+void launch_fwd_shape(const AttnParams& prm, int64_t batch, hipStream_t st) {
+    constexpr int kBlockQ = FwdShape<HD, W>::kBlockQ;
+    const dim3 grid((unsigned)prm.hq, (unsigned)((prm.seq + kBlockQ - 1) / kBlockQ), (unsigned)batch);
+    hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, HD, W>), grid, dim3(64 * W), 0, st, prm);
 }
 
-// An odd number of 128-query blocks takes 4-wave blocks at head_dim 128,
-// except for the packed FP16 exp2 programs: their 4-wave kernels would spill
-// (both lanes of each packed pair stay live: up to 17 registers at routes 4
-// and 6), so they run the 8-wave ragged kernel, whose last block holds 128
-// queries past the sequence that load the last row and store nothing.
+// Waves per head_dim-128 block.  One 8-wave block per CU stages each tile once
+// for 256 queries and is the faster shape where its blocks fill the CUs
+// evenly: an even number of whole rounds (causal blocks are dispatched
+// heaviest first, so two rounds add up to equal loads), or many rounds.
+// Anything else ends in a round that leaves CUs idle, and two 4-wave blocks
+// per CU, half the size, lose less.  Causal, 32 heads, hardware softmax /
+// softcap D4, 8 against 4 waves: S 4096 (two rounds) 151 / 221 against 156 /
+// 238 us; S 6001 (three) 314 / 487 against 299 / 461; S 2048 (one) 65 / 104
+// against 59 / 85.
+int fwd_waves(const AttnParams& prm, int64_t batch) {
+    const int64_t blocks = batch * prm.hq * ((prm.seq + 255) / 256), cus = device_shape().cus;
+    return blocks % (2 * cus) == 0 || blocks >= 10 * cus ? 8 : 4;
+}
+
 template <int MODE, int ROUTE>
-void launch_fwd(const AttnParams& prm, dim3 grid, hipStream_t st, int hd) {
-    if (hd == 64) {
-        launch_fwd_shape<MODE, ROUTE, 64, 4>(prm, grid, st);
-    } else if constexpr (fwd_program_heavy<MODE>()) {
-        launch_fwd_shape<MODE, ROUTE, 128, 4>(prm, grid, st);
-    } else if (grid.y % 2 == 0) {
-        launch_fwd_shape<MODE, ROUTE, 128, 8>(prm, dim3(grid.x, grid.y / 2, grid.z), st);
-    } else if constexpr (exp2_is_f16(attn_exp2_kind<MODE>())) {
-        hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, 128, 8, true>), dim3(grid.x, (grid.y + 1) / 2, grid.z),
-                           dim3(64 * 8), 0, st, prm);
-    } else {
-        launch_fwd_shape<MODE, ROUTE, 128, 4>(prm, grid, st);
-    }
+void launch_fwd(const AttnParams& prm, int64_t batch, hipStream_t st, int hd) {
+    if (hd == 64) launch_fwd_shape<MODE, ROUTE, 64, 4>(prm, batch, st);
+    else if (fwd_waves(prm, batch) == 8) launch_fwd_shape<MODE, ROUTE, 128, 8>(prm, batch, st);
+    else launch_fwd_shape<MODE, ROUTE, 128, 4>(prm, batch, st);
 }
 
 template <int MODE>
-void launch_routed(const AttnParams& prm, dim3 grid, hipStream_t st, int route, int hd) {
+void launch_routed(const AttnParams& prm, int64_t batch, hipStream_t st, int route, int hd) {
     switch (route) {
-        case 6: launch_fwd<MODE, 6>(prm, grid, st, hd); break;
-        case 8: launch_fwd<MODE, 8>(prm, grid, st, hd); break;
-        case 10: launch_fwd<MODE, 10>(prm, grid, st, hd); break;
-        case 12: launch_fwd<MODE, 12>(prm, grid, st, hd); break;
-        case 16: launch_fwd<MODE, 16>(prm, grid, st, hd); break;
-        case 20: launch_fwd<MODE, 20>(prm, grid, st, hd); break;
-        case 24: launch_fwd<MODE, 24>(prm, grid, st, hd); break;
-        case 32: launch_fwd<MODE, 32>(prm, grid, st, hd); break;
-        case 4: launch_fwd<MODE, 4>(prm, grid, st, hd); break;
-        default: launch_fwd<MODE, kRouteRuntime>(prm, grid, st, hd); break;
+        case 6: launch_fwd<MODE, 6>(prm, batch, st, hd); break;
+        case 8: launch_fwd<MODE, 8>(prm, batch, st, hd); break;
+        case 10: launch_fwd<MODE, 10>(prm, batch, st, hd); break;
+        case 12: launch_fwd<MODE, 12>(prm, batch, st, hd); break;
+        case 16: launch_fwd<MODE, 16>(prm, batch, st, hd); break;
+        case 20: launch_fwd<MODE, 20>(prm, batch, st, hd); break;
+        case 24: launch_fwd<MODE, 24>(prm, batch, st, hd); break;
+        case 32: launch_fwd<MODE, 32>(prm, batch, st, hd); break;
+        case 4: launch_fwd<MODE, 4>(prm, batch, st, hd); break;
+        default: launch_fwd<MODE, kRouteRuntime>(prm, batch, st, hd); break;
     }
 }
 
@@ -585,46 +617,48 @@ extern "C" int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* ls
     if (batch > 65535 || qblocks > 65535 || q_heads > 0x7fffffff) return hipErrorInvalidValue;
     AttnParams prm{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out, lse,
                    st[0], st[1], st[2], st[3], q_heads, kv_heads, seq, valid_keys, scale,
-                   cap > 0.0f ? cap : 1.0f, sigmoid_bias, causal != 0, exp2_route, host_route_mask(exp2_route)};
-    const dim3 grid((unsigned)q_heads, (unsigned)qblocks, (unsigned)batch);
+                   cap > 0.0f ? cap : 1.0f, sigmoid_bias, causal != 0, exp2_route, host_route_mask(exp2_route),
+                   (int)(q_heads / kv_heads), 0};
+    // staging adds up to 7 rows to a wave's address as a 32-bit byte offset
+    for (int i = 0; i < 3; ++i) prm.wide |= st[i].s > (int64_t(1) << 27);
     hipStream_t hst = hs(stream);
     switch (mode) {
-        case kAttnSoftmaxNative: launch_fwd<kAttnSoftmaxNative, 0>(prm, grid, hst, hd); break;
-        case kAttnSoftmaxExp2D2: launch_routed<kAttnSoftmaxExp2D2>(prm, grid, hst, exp2_route, hd); break;
-        case kAttnSoftmaxExp2D3: launch_routed<kAttnSoftmaxExp2D3>(prm, grid, hst, exp2_route, hd); break;
-        case kAttnSoftmaxExp2Pwl2: launch_routed<kAttnSoftmaxExp2Pwl2>(prm, grid, hst, exp2_route, hd); break;
+        case kAttnSoftmaxNative: launch_fwd<kAttnSoftmaxNative, 0>(prm, batch, hst, hd); break;
+        case kAttnSoftmaxExp2D2: launch_routed<kAttnSoftmaxExp2D2>(prm, batch, hst, exp2_route, hd); break;
+        case kAttnSoftmaxExp2D3: launch_routed<kAttnSoftmaxExp2D3>(prm, batch, hst, exp2_route, hd); break;
+        case kAttnSoftmaxExp2Pwl2: launch_routed<kAttnSoftmaxExp2Pwl2>(prm, batch, hst, exp2_route, hd); break;
         case kAttnSoftmaxExp2Pwl2Safe:
-            launch_routed<kAttnSoftmaxExp2Pwl2Safe>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2Pwl2Safe>(prm, batch, hst, exp2_route, hd);
             break;
         case kAttnSoftmaxExp2Pwl2SafeF16:
-            launch_routed<kAttnSoftmaxExp2Pwl2SafeF16>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2Pwl2SafeF16>(prm, batch, hst, exp2_route, hd);
             break;
-        case kAttnSoftmaxExp2Pwl1Safe: launch_routed<kAttnSoftmaxExp2Pwl1Safe>(prm, grid, hst, exp2_route, hd); break;
+        case kAttnSoftmaxExp2Pwl1Safe: launch_routed<kAttnSoftmaxExp2Pwl1Safe>(prm, batch, hst, exp2_route, hd); break;
         case kAttnSoftmaxExp2Pwl1SafeF16:
-            launch_routed<kAttnSoftmaxExp2Pwl1SafeF16>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2Pwl1SafeF16>(prm, batch, hst, exp2_route, hd);
             break;
         case kAttnSoftmaxExp2Pwl2SafeBF16:
-            launch_routed<kAttnSoftmaxExp2Pwl2SafeBF16>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2Pwl2SafeBF16>(prm, batch, hst, exp2_route, hd);
             break;
         case kAttnSoftmaxExp2D2NoClamp:
-            launch_routed<kAttnSoftmaxExp2D2NoClamp>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2D2NoClamp>(prm, batch, hst, exp2_route, hd);
             break;
         case kAttnSoftmaxExp2D2SafeF16:
-            launch_routed<kAttnSoftmaxExp2D2SafeF16>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2D2SafeF16>(prm, batch, hst, exp2_route, hd);
             break;
         case kAttnSoftmaxExp2D2SafeBF16:
-            launch_routed<kAttnSoftmaxExp2D2SafeBF16>(prm, grid, hst, exp2_route, hd);
+            launch_routed<kAttnSoftmaxExp2D2SafeBF16>(prm, batch, hst, exp2_route, hd);
             break;
-        case kAttnSoftmaxExp2Pwl2F16: launch_routed<kAttnSoftmaxExp2Pwl2F16>(prm, grid, hst, exp2_route, hd); break;
-        case kAttnSoftcapNative: launch_fwd<kAttnSoftcapNative, 0>(prm, grid, hst, hd); break;
-        case kAttnSoftcapD4: launch_fwd<kAttnSoftcapD4, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidNative: launch_fwd<kAttnSigmoidNative, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidB3: launch_fwd<kAttnSigmoidB3, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidB3D2: launch_fwd<kAttnSigmoidB3D2, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidD3: launch_fwd<kAttnSigmoidD3, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidD3 + 1: launch_fwd<kAttnSigmoidD3 + 1, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidD3 + 2: launch_fwd<kAttnSigmoidD3 + 2, 0>(prm, grid, hst, hd); break;
-        case kAttnSigmoidD6: launch_fwd<kAttnSigmoidD6, 0>(prm, grid, hst, hd); break;
+        case kAttnSoftmaxExp2Pwl2F16: launch_routed<kAttnSoftmaxExp2Pwl2F16>(prm, batch, hst, exp2_route, hd); break;
+        case kAttnSoftcapNative: launch_fwd<kAttnSoftcapNative, 0>(prm, batch, hst, hd); break;
+        case kAttnSoftcapD4: launch_fwd<kAttnSoftcapD4, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidNative: launch_fwd<kAttnSigmoidNative, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidB3: launch_fwd<kAttnSigmoidB3, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidB3D2: launch_fwd<kAttnSigmoidB3D2, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidD3: launch_fwd<kAttnSigmoidD3, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidD3 + 1: launch_fwd<kAttnSigmoidD3 + 1, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidD3 + 2: launch_fwd<kAttnSigmoidD3 + 2, 0>(prm, batch, hst, hd); break;
+        case kAttnSigmoidD6: launch_fwd<kAttnSigmoidD6, 0>(prm, batch, hst, hd); break;
     }
     return hipGetLastError();
 }

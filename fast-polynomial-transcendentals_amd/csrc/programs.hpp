@@ -67,11 +67,10 @@ __device__ __forceinline__ float bf_hi(uint32_t u) { return as_f32(u & 0xffff000
 
 // Round an FP32 value to BF16 (RNE) and return it as FP32: one
 // v_cvt_pk_bf16_f32 that writes bf16(x) to the high half and bf16(0) = 0 to
-// the low half.
+// the low half (the conversion of {0, x}; as inline asm the same instruction
+// drew a wait state before most of its uses).
 __device__ __forceinline__ float rbf(float x) {
-    float r;
-    asm("v_cvt_pk_bf16_f32 %0, 0, %1" : "=v"(r) : "v"(x));
-    return r;
+    return __builtin_bit_cast(float, __builtin_convertvector((f2_t){0.0f, x}, bf2_t));
 }
 
 // Pack two FP32 values into a BF16 pair with RNE.
@@ -379,6 +378,17 @@ struct BF16Prog {
         return h;
     }
 
+    // The same with the coefficients (BF16 values, c[1..deg]) in registers:
+    // a loop that keeps them in VGPRs issues its FMAs at twice the rate of
+    // ones with a scalar operand (2.6 against 4.5 cycles per wave, measured
+    // with two waves per SIMD).
+    __device__ __forceinline__ static float odd_horner(float t, const float (&c)[P.deg + 1]) {
+        float h = bfma(t, c[P.deg], c[P.deg - 1]);
+#pragma unroll
+        for (int i = P.deg - 2; i >= 1; --i) h = bfma(t, h, c[i]);
+        return h;
+    }
+
     // Even programs, up to the final rounding; t is the clamped magnitude.
     __device__ __forceinline__ static float even_open(float t) {
         float r = bfma(t, bf16_value(P.c[P.deg]), bf16_value(P.c[P.deg - 1]));
@@ -392,7 +402,9 @@ struct BF16Prog {
     // the last product ts*H(|ts|) is sign(x)*t*H(t) exactly, so no separate
     // sign restore is needed.
     __device__ __forceinline__ static float odd_signed_open(float ts) {
-        const float v = ts * odd_horner(__builtin_fabsf(ts));
+        return odd_signed_close(ts * odd_horner(__builtin_fabsf(ts)));
+    }
+    __device__ __forceinline__ static float odd_signed_close(float v) {
         if constexpr (P.shape == kOdd) {
             return v;
         } else if constexpr (P.shape == kOddMin1) {
@@ -447,6 +459,15 @@ struct BF16Prog {
         open2(x, ol, oh);
         lo = rbf(ol);
         hi = rbf(oh);
+    }
+
+    // eval2 of the odd shapes with the coefficients in registers.
+    __device__ __forceinline__ static void eval2(uint32_t x, const float (&c)[P.deg + 1], float& lo, float& hi) {
+        static_assert(P.shape == kOdd || P.shape == kOddMin1, "an odd program");
+        const uint32_t ts = sclamp16x2(x, bf16_pair_bits(P.lc));
+        const float l = bf_lo(ts), h = bf_hi(ts);
+        lo = rbf(odd_signed_close(l * odd_horner(__builtin_fabsf(l), c)));
+        hi = rbf(odd_signed_close(h * odd_horner(__builtin_fabsf(h), c)));
     }
 
     __device__ __forceinline__ static uint32_t eval(uint32_t x) {

@@ -67,15 +67,19 @@ __device__ __forceinline__ h2_t b3_row_pair(bool row, uint32_t w0, uint32_t w1) 
 // semantics: the clamp keeps NaN, max(0, NaN) gives 0, the derivative is NaN.
 // OPEN_Y (probability only) returns y before its final rounding, for callers
 // whose conversion to BF16 is that rounding: RNE of an already rounded value
-// is the same value, so the converted bits are unchanged.
-template <bool WITH_GRAD, bool OPEN_Y = false>
+// is the same value, so the converted bits are unchanged.  QUIET_X: x is no
+// signaling NaN.
+template <bool WITH_GRAD, bool OPEN_Y = false, bool QUIET_X = false>
 __device__ __forceinline__ void b3_lane(float x, float& y, float& dy) {
     static_assert(!(WITH_GRAD && OPEN_Y), "the derivative multiplies the rounded probability");
     using C = B3Consts;
     using P = B3Pairs;
     const bool row = x >= C::split;
-    const float xc = __builtin_elementwise_minimum(
-        __builtin_elementwise_maximum(x, -C::clamp), C::clamp);
+    // v_med3_f32 clamps a quiet NaN to -6, and y(-6) is 0 as y(NaN) is, so the
+    // probability of a score that arithmetic produced needs one instruction
+    // (a signaling NaN clamps to 6)
+    const float xc = QUIET_X && !WITH_GRAD ? __builtin_amdgcn_fmed3f(x, -C::clamp, C::clamp)
+                                           : __builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -C::clamp), C::clamp);
     const h2_t c32 = b3_row_pair(row, P::c32_0, P::c32_1);
     const h2_t c10 = b3_row_pair(row, P::c10_0, P::c10_1);
     float f = bfma(xc, (float)c32.y, (float)c32.x);

@@ -584,8 +584,8 @@ int launch_flash_attention_fwd_strided_bf16(void* out, float* lse, const void* q
 /* The same forward with keys valid_keys .. seq - 1 masked as padding
  * (1 <= valid_keys <= seq), for callers that keep operands padded at the end
  * (the padded queries' rows are computed and left to the caller to drop).
- * The padded K and V rows are zeroed on chip before use, so they may hold
- * anything (NaN and Inf included).  The padded queries attend to the valid
+ * The padded K and V rows are never read, so they may hold anything (NaN
+ * and Inf included).  The padded queries attend to the valid
  * keys: their out rows and lse are finite for finite Q rows.
  * The backward takes no valid_keys.  It serves padded operands when the
  * padded K rows are zero, the padded V, Q and out rows finite and the padded
