@@ -670,9 +670,7 @@ void check_attn_operand(const at::Tensor& t, const char* name) {
     TORCH_CHECK(t.stride(3) == 1, name, " must be contiguous in head_dim");
 }
 
-std::vector<at::Tensor> flash_attn_fwd_bf16(at::Tensor q, at::Tensor k, at::Tensor v, int64_t mode,
-                                            int64_t exp2_route, bool causal, double softmax_scale,
-                                            double softcap, double sigmoid_bias, int64_t valid_keys) {
+void check_attn_fwd(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v) {
     check_attn_operand(q, "q");
     check_attn_operand(k, "k");
     check_attn_operand(v, "v");
@@ -682,16 +680,26 @@ std::vector<at::Tensor> flash_attn_fwd_bf16(at::Tensor q, at::Tensor k, at::Tens
     TORCH_CHECK(q.size(3) == 64 || q.size(3) == 128, "head_dim must be 64 or 128, got ", q.size(3));
     TORCH_CHECK(q.size(2) % k.size(2) == 0, "q heads (", q.size(2),
                 ") must be a multiple of kv heads (", k.size(2), ")");
+}
+
+// lse [B, Hq, S]: the softmax and softcap modes write every row; the sigmoid
+// modes (5..11) have no partition function and leave it untouched, so only
+// they need it cleared
+at::Tensor empty_lse(const at::Tensor& q, int64_t mode) {
+    const auto options = q.options().dtype(at::kFloat);
+    return mode >= 5 && mode <= 11 ? at::zeros({q.size(0), q.size(2), q.size(1)}, options)
+                                   : at::empty({q.size(0), q.size(2), q.size(1)}, options);
+}
+
+std::vector<at::Tensor> flash_attn_fwd_bf16(at::Tensor q, at::Tensor k, at::Tensor v, int64_t mode,
+                                            int64_t exp2_route, bool causal, double softmax_scale,
+                                            double softcap, double sigmoid_bias, int64_t valid_keys) {
+    check_attn_fwd(q, k, v);
     c10::OptionalDeviceGuard guard(q.device());
     const int64_t b = q.size(0), sq = q.size(1), hq = q.size(2), hkv = k.size(2);
     const int64_t d = q.size(3);
     at::Tensor out = at::empty({b, sq, hq, d}, q.options());
-    // the softmax and softcap modes write every lse row; the sigmoid modes
-    // (5..11) have no partition function and leave it untouched, so only
-    // they need it cleared
-    const bool sigmoid_mode = mode >= 5 && mode <= 11;
-    at::Tensor lse = sigmoid_mode ? at::zeros({b, hq, sq}, q.options().dtype(at::kFloat))
-                                  : at::empty({b, hq, sq}, q.options().dtype(at::kFloat));
+    at::Tensor lse = empty_lse(q, mode);
     const int64_t strides[12] = {q.stride(0), q.stride(2), q.stride(1), k.stride(0), k.stride(2),
                                  k.stride(1), v.stride(0), v.stride(2), v.stride(1), out.stride(0),
                                  out.stride(2), out.stride(1)};
@@ -705,6 +713,37 @@ std::vector<at::Tensor> flash_attn_fwd_bf16(at::Tensor q, at::Tensor k, at::Tens
                      (float)sigmoid_bias, s),
                  s);
     return {out, lse};
+}
+
+// O in the layout of a (batch, heads, sequence, dim) caller, written by the
+// kernel in place of a transposing copy behind it; with keep also what the
+// backward takes, O [B, S, Hq, D] (its own memory: the caller may edit the
+// first) and lse.
+std::vector<at::Tensor> flash_attn_fwd_heads_first_bf16(at::Tensor q, at::Tensor k, at::Tensor v, int64_t mode,
+                                                        int64_t exp2_route, bool causal, double softmax_scale,
+                                                        double softcap, double sigmoid_bias, bool keep) {
+    check_attn_fwd(q, k, v);
+    c10::OptionalDeviceGuard guard(q.device());
+    const int64_t b = q.size(0), sq = q.size(1), hq = q.size(2), hkv = k.size(2), d = q.size(3);
+    at::Tensor first = at::empty({b, hq, sq, d}, q.options()), out, lse;
+    int64_t strides[15] = {q.stride(0), q.stride(2), q.stride(1), k.stride(0), k.stride(2),
+                           k.stride(1), v.stride(0), v.stride(2), v.stride(1), hq * sq * d, sq * d, d};
+    if (keep) {
+        out = at::empty({b, sq, hq, d}, q.options());
+        lse = empty_lse(q, mode);
+        strides[12] = sq * hq * d;
+        strides[13] = d;
+        strides[14] = hq * d;
+    }
+    void* s = current_stream(q);
+    check_launch(launch_flash_attention_fwd_two_outputs_bf16(
+                     first.data_ptr(), keep ? out.data_ptr() : nullptr, keep ? lse.data_ptr<float>() : nullptr,
+                     q.data_ptr(), k.data_ptr(), v.data_ptr(), b, hq, hkv, sq, sq, d, strides, (int)mode,
+                     (int)exp2_route, causal ? 1 : 0, (float)softmax_scale, (float)softcap,
+                     (float)sigmoid_bias, s),
+                 s);
+    if (keep) return {first, out, lse};
+    return {first};
 }
 
 // Largest dS workspace the attention backward allocates: the environment's
@@ -1396,6 +1435,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           "Fused attention forward with the score programs in the tile loop; "
           "q [B,S,Hq,D], k/v [B,S,Hkv,D] BF16 (D 64 or 128, any S) -> [out [B,S,Hq,D], lse [B,Hq,S] FP32]; "
           "valid_keys >= 1 masks keys from that index on (operands padded at the end)");
+    m.def("flash_attn_fwd_heads_first_bf16", &flash_attn_fwd_heads_first_bf16, py::arg("q"), py::arg("k"),
+          py::arg("v"), py::arg("mode"), py::arg("exp2_route") = 4, py::arg("causal") = true,
+          py::arg("softmax_scale"), py::arg("softcap") = 0.0, py::arg("sigmoid_bias") = 0.0,
+          py::arg("keep") = true,
+          "flash_attn_fwd_bf16 of the same operands -> [out [B,Hq,S,D]], with keep followed by "
+          "out [B,S,Hq,D] and lse [B,Hq,S] for the backward");
     m.def("flash_attn_bwd_bf16", &flash_attn_bwd_bf16, py::arg("q"), py::arg("k"), py::arg("v"),
           py::arg("out"), py::arg("dout"), py::arg("lse"), py::arg("mode"), py::arg("grad") = 0,
           py::arg("exp2_route") = 0, py::arg("causal") = true, py::arg("softmax_scale"),

@@ -55,8 +55,9 @@ struct AttnParams {
     const uint16_t* k;
     const uint16_t* v;
     uint16_t* o;
+    uint16_t* o2;  // the same rows at strides o2s, or null
     float* lse;  // [B, Hq, S] natural-log partition function, or null
-    AttnStrides qs, ks, vs, os;
+    AttnStrides qs, ks, vs, os, o2s;
     int64_t hq, hkv, seq;
     int64_t kv_len;  // keys 0 .. kv_len - 1 are real, the rest padding (masked)
     float scale;     // s = q.k * scale
@@ -519,12 +520,16 @@ __global__ void __launch_bounds__(64 * W)
                           pack_bf(oacc[dt][4 * g + 2] * inv, oacc[dt][4 * g + 3] * inv)};
     __builtin_amdgcn_wave_barrier();  // LDS accesses of one wave complete in order
     uint16_t* op = p.o + b * p.os.b + head * p.os.h;
+    uint16_t* o2p = p.o2 != nullptr ? p.o2 + b * p.o2s.b + head * p.o2s.h : nullptr;
 #pragma unroll
     for (int j = 0; j < 32 / F::kLoadRows; ++j) {
         const int r = j * F::kLoadRows + loader.lr;
         const u32x4_t w =
             *reinterpret_cast<const u32x4_t*>(orows + r * kRowB + (loader.lc ^ (r & (F::kChunks - 1))) * 16);
-        if (q0 + r < seq) *reinterpret_cast<u32x4_t*>(op + (q0 + r) * p.os.s + loader.lc * 8) = w;
+        if (q0 + r < seq) {
+            *reinterpret_cast<u32x4_t*>(op + (q0 + r) * p.os.s + loader.lc * 8) = w;
+            if (o2p != nullptr) *reinterpret_cast<u32x4_t*>(o2p + (q0 + r) * p.o2s.s + loader.lc * 8) = w;
+        }
     }
 }
 
@@ -586,13 +591,13 @@ bool stride_ok(const AttnStrides& t) { return t.b >= 0 && t.h >= 0 && t.s >= 0 &
 
 }  // namespace
 
-extern "C" int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* lse, const void* q,
-                                                            const void* k, const void* v, int64_t batch,
-                                                            int64_t q_heads, int64_t kv_heads, int64_t seq,
-                                                            int64_t valid_keys, int64_t head_dim,
-                                                            const int64_t* strides, int mode, int exp2_route,
-                                                            int causal, float scale, float cap,
-                                                            float sigmoid_bias, void* stream) {
+extern "C" int launch_flash_attention_fwd_two_outputs_bf16(void* out, void* out2, float* lse, const void* q,
+                                                           const void* k, const void* v, int64_t batch,
+                                                           int64_t q_heads, int64_t kv_heads, int64_t seq,
+                                                           int64_t valid_keys, int64_t head_dim,
+                                                           const int64_t* strides, int mode, int exp2_route,
+                                                           int causal, float scale, float cap,
+                                                           float sigmoid_bias, void* stream) {
     if (batch < 0 || q_heads <= 0 || kv_heads <= 0 || seq < 0 || (head_dim != 64 && head_dim != 128) || !strides)
         return hipErrorInvalidValue;
     if (seq > 0 && (valid_keys < 1 || valid_keys > seq)) return hipErrorInvalidValue;
@@ -608,15 +613,19 @@ extern "C" int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* ls
                                {strides[6], strides[7], strides[8]}, {strides[9], strides[10], strides[11]}};
     for (const AttnStrides& t : st)
         if (!stride_ok(t)) return hipErrorInvalidValue;
+    AttnStrides st2{};
+    if (out2) st2 = {strides[12], strides[13], strides[14]};
+    if (!stride_ok(st2)) return hipErrorInvalidValue;
     if (batch == 0 || seq == 0) return hipSuccess;
     if (!out || !q || !k || !v || !aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v))
         return hipErrorInvalidValue;
+    if (out2 && !aligned16(out2)) return hipErrorInvalidValue;
     if (lse && (reinterpret_cast<uintptr_t>(lse) & 3)) return hipErrorInvalidValue;
     if (attn_is_sigmoid(mode)) lse = nullptr;  // sigmoid attention has no partition function
     const int64_t qblocks = (seq + kAttnBlockQ - 1) / kAttnBlockQ;  // the last one may be partial
     if (batch > 65535 || qblocks > 65535 || q_heads > 0x7fffffff) return hipErrorInvalidValue;
-    AttnParams prm{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out, lse,
-                   st[0], st[1], st[2], st[3], q_heads, kv_heads, seq, valid_keys, scale,
+    AttnParams prm{(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (uint16_t*)out,
+                   (uint16_t*)out2, lse, st[0], st[1], st[2], st[3], st2, q_heads, kv_heads, seq, valid_keys, scale,
                    cap > 0.0f ? cap : 1.0f, sigmoid_bias, causal != 0, exp2_route, host_route_mask(exp2_route),
                    (int)(q_heads / kv_heads), 0};
     // staging adds up to 7 rows to a wave's address as a 32-bit byte offset
@@ -661,6 +670,18 @@ extern "C" int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* ls
         case kAttnSigmoidD6: launch_fwd<kAttnSigmoidD6, 0>(prm, batch, hst, hd); break;
     }
     return hipGetLastError();
+}
+
+extern "C" int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* lse, const void* q,
+                                                            const void* k, const void* v, int64_t batch,
+                                                            int64_t q_heads, int64_t kv_heads, int64_t seq,
+                                                            int64_t valid_keys, int64_t head_dim,
+                                                            const int64_t* strides, int mode, int exp2_route,
+                                                            int causal, float scale, float cap,
+                                                            float sigmoid_bias, void* stream) {
+    return launch_flash_attention_fwd_two_outputs_bf16(out, nullptr, lse, q, k, v, batch, q_heads, kv_heads, seq,
+                                                       valid_keys, head_dim, strides, mode, exp2_route, causal,
+                                                       scale, cap, sigmoid_bias, stream);
 }
 
 extern "C" int launch_flash_attention_fwd_strided_bf16(void* out, float* lse, const void* q,

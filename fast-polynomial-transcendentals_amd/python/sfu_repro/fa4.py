@@ -464,14 +464,21 @@ class _FA4Function(torch.autograd.Function):
                 sigmoid_sfu_res, sigmoid_sfu_freq_bwd, sigmoid_sfu_res_bwd, sigmoid_use_direct_bwd_poly,
                 sigmoid_bias, sigmoid_poly_backend, sigmoid_degree, sigmoid_degree_bwd, sigmoid_coeff_source,
                 exp2_emu_backend, exp2_emu_freq, exp2_emu_freq_bwd, score_mod, score_mod_bwd, flash_attn_fwd,
-                flash_attn_bwd):
+                flash_attn_bwd, heads_first, keep):
         fused_softcap = softcap if score_mod is None else 0.0
-        out, lse = flash_attn_fwd(
-            q, k, v, softmax_scale=softmax_scale, causal=causal, softcap=fused_softcap, score_mod=score_mod,
+        kw = dict(
+            softmax_scale=softmax_scale, causal=causal, softcap=fused_softcap, score_mod=score_mod,
             sigmoid_attention=sigmoid_attention, sigmoid_sfu_freq=sigmoid_sfu_freq,
             sigmoid_sfu_res=sigmoid_sfu_res, sigmoid_bias=sigmoid_bias, sigmoid_poly_backend=sigmoid_poly_backend,
             sigmoid_degree=sigmoid_degree, sigmoid_coeff_source=sigmoid_coeff_source,
             exp2_emu_backend=exp2_emu_backend, exp2_emu_freq=exp2_emu_freq)
+        if heads_first is None:
+            out, lse = flash_attn_fwd(q, k, v, **kw)
+            result = out
+        else:
+            result, out, lse = heads_first(q, k, v, keep=keep, **kw)
+            if not keep:
+                return result
         ctx.save_for_backward(q, k, v, out, lse)
         ctx.kw = dict(
             softmax_scale=softmax_scale, causal=causal, softcap=fused_softcap, score_mod=score_mod,
@@ -485,25 +492,42 @@ class _FA4Function(torch.autograd.Function):
             sigmoid_coeff_source=sigmoid_coeff_source, exp2_emu_backend=exp2_emu_backend,
             exp2_emu_freq=exp2_emu_freq_bwd)
         ctx.flash_attn_bwd = flash_attn_bwd
-        return out
+        ctx.heads_first = heads_first is not None
+        return result
 
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out, lse = ctx.saved_tensors
         kw = dict(ctx.kw)
         softmax_scale, causal, softcap = kw.pop("softmax_scale"), kw.pop("causal"), kw.pop("softcap")
-        dq, dk, dv = ctx.flash_attn_bwd(q, k, v, out, dout.contiguous(), lse, softmax_scale, causal, softcap, **kw)
-        return (dq, dk, dv) + (None,) * 21
+        if ctx.heads_first:
+            # the kernels read the gradient where it lies (a copy to the
+            # operands' layout took 26 us of a 740 us step at 32 heads, 4096
+            # rows, head_dim 128); 16-byte loads need its alignment
+            lies_well = dout.is_contiguous() and dout.data_ptr() % 16 == 0
+            dout = dout.transpose(1, 2) if lies_well else dout.transpose(1, 2).contiguous()
+        else:
+            dout = dout.contiguous()
+        dq, dk, dv = ctx.flash_attn_bwd(q, k, v, out, dout, lse, softmax_scale, causal, softcap, **kw)
+        return (dq, dk, dv) + (None,) * 23
 
 
 def _fa4(q, k, v, *, softmax_scale: float | None, causal: bool, config: ResolvedFA4Config) -> torch.Tensor:
-    return _FA4Function.apply(
+    """q, k, v (batch, sequence, heads, dim) -> out (batch, heads, sequence,
+    dim), contiguous.  This package's kernels store it so; for another
+    runtime's it is copied."""
+    from . import fa4_runtime
+
+    own = config.flash_attn_fwd is fa4_runtime.flash_attn_fwd and config.flash_attn_bwd is fa4_runtime.flash_attn_bwd
+    keep = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    out = _FA4Function.apply(
         q, k, v, softmax_scale, causal, config.softcap, config.sigmoid_attention, config.sigmoid_sfu_freq,
         config.sigmoid_sfu_res, config.sigmoid_sfu_freq_bwd, config.sigmoid_sfu_res_bwd,
         config.sigmoid_use_direct_bwd_poly, config.sigmoid_bias, config.sigmoid_poly_backend,
         config.sigmoid_degree, config.sigmoid_degree_bwd, config.sigmoid_coeff_source, config.exp2_emu_backend,
         config.exp2_emu_freq, config.exp2_emu_freq_bwd, config.score_mod, config.score_mod_bwd,
-        config.flash_attn_fwd, config.flash_attn_bwd)
+        config.flash_attn_fwd, config.flash_attn_bwd, fa4_runtime.flash_attn_fwd_heads_first if own else None, keep)
+    return out if own else out.transpose(1, 2).contiguous()
 
 
 class FA4AttentionWrapper(nn.Module):
@@ -531,9 +555,8 @@ class FA4AttentionWrapper(nn.Module):
         if self.q_norm is not None:
             q, k = self.q_norm(q), self.k_norm(k)
         dtype = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else q.dtype
-        out = _fa4(q.transpose(1, 2).contiguous().to(dtype), k.transpose(1, 2).contiguous().to(dtype),
-                   v.transpose(1, 2).contiguous().to(dtype), softmax_scale=scale, causal=True, config=self.config)
-        return out.transpose(1, 2).contiguous()
+        return _fa4(q.transpose(1, 2).contiguous().to(dtype), k.transpose(1, 2).contiguous().to(dtype),
+                    v.transpose(1, 2).contiguous().to(dtype), softmax_scale=scale, causal=True, config=self.config)
 
 
 def build_fa4_module(config: FA4Config, *, head_dim: int, sequence_length: int | None = None) -> FA4AttentionWrapper:

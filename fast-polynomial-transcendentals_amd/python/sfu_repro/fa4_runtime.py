@@ -326,11 +326,12 @@ def _check_operands(q, k, v):
             raise ValueError(f"{name} must be [batch, seqlen, heads, head_dim]")
 
 
-def flash_attn_fwd(q, k, v, softmax_scale=None, causal=False, softcap=0.0, score_mod=None,
-                   sigmoid_attention=False, sigmoid_sfu_freq=16, sigmoid_sfu_res=0, sigmoid_bias=None,
-                   sigmoid_poly_backend="cute", sigmoid_degree=3, sigmoid_coeff_source="current",
-                   exp2_emu_backend="d3", exp2_emu_freq=None, **unused):
-    """FA4's forward: returns (out [B, S, Hq, D], lse [B, Hq, S])."""
+def _forward_arguments(q, k, v, softmax_scale=None, causal=False, softcap=0.0, score_mod=None,
+                       sigmoid_attention=False, sigmoid_sfu_freq=16, sigmoid_sfu_res=0, sigmoid_bias=None,
+                       sigmoid_poly_backend="cute", sigmoid_degree=3, sigmoid_coeff_source="current",
+                       exp2_emu_backend="d3", exp2_emu_freq=None, **unused):
+    """The forward kernels' arguments behind the operands, for
+    :func:`flash_attn_fwd`'s arguments."""
     if unused:
         raise TypeError("unsupported flash_attn_fwd arguments: " + ", ".join(sorted(unused)))
     _check_operands(q, k, v)
@@ -343,7 +344,28 @@ def flash_attn_fwd(q, k, v, softmax_scale=None, causal=False, softcap=0.0, score
         exp2_emu_freq=exp2_emu_freq)
     if q.shape[1] < 1:
         raise ValueError(f"seqlen must be positive, got {q.shape[1]}")
-    return tuple(_ops().flash_attn_fwd_bf16(q, k, v, mode, route, bool(causal), scale, cap, bias))
+    return mode, route, bool(causal), scale, cap, bias
+
+
+def flash_attn_fwd(q, k, v, softmax_scale=None, causal=False, softcap=0.0, score_mod=None,
+                   sigmoid_attention=False, sigmoid_sfu_freq=16, sigmoid_sfu_res=0, sigmoid_bias=None,
+                   sigmoid_poly_backend="cute", sigmoid_degree=3, sigmoid_coeff_source="current",
+                   exp2_emu_backend="d3", exp2_emu_freq=None, **unused):
+    """FA4's forward: returns (out [B, S, Hq, D], lse [B, Hq, S])."""
+    args = _forward_arguments(
+        q, k, v, softmax_scale, causal, softcap, score_mod, sigmoid_attention, sigmoid_sfu_freq, sigmoid_sfu_res,
+        sigmoid_bias, sigmoid_poly_backend, sigmoid_degree, sigmoid_coeff_source, exp2_emu_backend, exp2_emu_freq,
+        **unused)
+    return tuple(_ops().flash_attn_fwd_bf16(q, k, v, *args))
+
+
+def flash_attn_fwd_heads_first(q, k, v, *, keep: bool, **kwargs):
+    """:func:`flash_attn_fwd` for a (batch, heads, sequence, dim) caller:
+    returns out [B, Hq, S, D] in the kernel's own stores, and with ``keep``
+    (out [B, S, Hq, D], lse) for the backward, else (None, None)."""
+    args = _forward_arguments(q, k, v, **kwargs)
+    first, *kept = _ops().flash_attn_fwd_heads_first_bf16(q, k, v, *args, keep)
+    return (first, *kept) if keep else (first, None, None)
 
 
 def flash_attn_bwd(q, k, v, out, dout, lse, softmax_scale=None, causal=False, softcap=0.0,

@@ -599,6 +599,17 @@ int launch_flash_attention_fwd_strided_keys_bf16(void* out, float* lse, const vo
                                                  int64_t head_dim, const int64_t* strides, int mode,
                                                  int exp2_route, int causal, float scale, float cap,
                                                  float sigmoid_bias, void* stream);
+/* The same forward writing its rows twice, to out and, unless out2 is null,
+ * to out2: a caller that returns O in one layout and keeps it for the
+ * backward in another needs no transposing copy.  strides: 15 element strides,
+ * those of out2 after the 12 of q, k, v and out (not read when out2 is null). */
+int launch_flash_attention_fwd_two_outputs_bf16(void* out, void* out2, float* lse, const void* q,
+                                                const void* k, const void* v, int64_t batch,
+                                                int64_t q_heads, int64_t kv_heads, int64_t seq,
+                                                int64_t valid_keys, int64_t head_dim,
+                                                const int64_t* strides, int mode, int exp2_route,
+                                                int causal, float scale, float cap, float sigmoid_bias,
+                                                void* stream);
 /* Backward of the same attention (the runtime behind FA4's flash_attn_bwd,
  * src/sfu_repro/fa4.py:430-461): dq [B, S, Hq, D], dk and dv [B, S, Hkv, D]
  * BF16 from q, k, v, out, dout (BF16) and the forward's lse (softmax modes).

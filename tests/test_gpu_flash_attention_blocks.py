@@ -49,3 +49,53 @@ def test_rows_past_32_bit_offsets(spline_ops, cuda, d):
         wide.copy_(t)
         got = _out(spline_ops, *(wide if j == i else s for j, s in enumerate((q, k, v))), "softmax_native", True)
         assert all(torch.equal(a, b) for a, b in zip(got, want)), ("qkv"[i], d)
+
+
+@pytest.mark.parametrize("mode", ["softmax_d2", "softcap_native", "sigmoid_d4"])
+@pytest.mark.parametrize("d,heads,seq", [(64, 6, 1), (64, 4, 200), (128, 4, 129), (128, 512, 33)])
+def test_heads_first_output(spline_ops, cuda, mode, d, heads, seq):
+    print(f"heads first {mode} d {d} heads {heads} seq {seq}", flush=True)
+    q, k, v = (t.to(cuda) for t in _inputs(2, heads, heads // 2, seq, d + seq, d=d)[:3])
+    args = (M[mode], 12, True, 1 / math.sqrt(d), 30.0, 0.0)
+    out, lse = spline_ops.flash_attn_fwd_bf16(q, k, v, *args)
+    first, kept, kept_lse = spline_ops.flash_attn_fwd_heads_first_bf16(q, k, v, *args, True)
+    (alone,) = spline_ops.flash_attn_fwd_heads_first_bf16(q, k, v, *args, False)
+    assert first.is_contiguous() and alone.is_contiguous()
+    for a in (first, alone):
+        assert torch.equal(a, out.transpose(1, 2))
+    assert torch.equal(kept, out) and torch.equal(kept_lse, lse)
+
+
+@pytest.mark.parametrize("own", [True, False])
+def test_wrapper_output_and_gradient_layouts(cuda, own):
+    """The module's output is contiguous and the caller's to edit, and the
+    gradients are the same from a contiguous, a transposed, a misaligned and
+    an expanded dout, by this package's kernels and by a runtime around them
+    (whose calls keep the copies)."""
+    from sfu_repro import fa4_runtime
+    from sfu_repro.fa4 import FA4AttentionWrapper, FA4Config, resolve_fa4_config
+
+    runtime = fa4_runtime.runtime()
+    if not own:
+        runtime["flash_attn_fwd"] = lambda *a, **kw: fa4_runtime.flash_attn_fwd(*a, **kw)
+    module = FA4AttentionWrapper(resolve_fa4_config(FA4Config(), runtime=runtime), 64)
+    q, k, v, do = (t.transpose(1, 2).contiguous().to(cuda) for t in _inputs(2, 4, 2, 130, 7, d=64))
+
+    def grads(dout, edit=False):
+        leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+        out = module(*leaves)
+        assert out.is_contiguous() and out.shape == q.shape
+        with torch.no_grad():
+            assert torch.equal(module(q, k, v), out)
+        if edit:
+            out.mul_(2)
+        return torch.autograd.grad(out, leaves, dout)
+
+    shifted = torch.empty(do.numel() + 1, dtype=do.dtype, device=cuda)[1:].view_as(do).copy_(do)
+    row = do[:1, :1].expand_as(do)
+    want = grads(do)
+    for name, got, ref in (("transposed", grads(do.transpose(1, 2).contiguous().transpose(1, 2)), want),
+                           ("misaligned", grads(shifted), want),
+                           ("expanded", grads(row), grads(row.contiguous())),
+                           ("edited", grads(do / 2, edit=True), want)):  # halves and doubles are exact
+        assert all(torch.equal(a, b) for a, b in zip(got, ref)), name
