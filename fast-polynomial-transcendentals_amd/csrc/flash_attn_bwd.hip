@@ -88,6 +88,8 @@ struct AttnBwdParams {
     int causal;
     int route;       // exp2 route of the kRouteRuntime instantiations
     uint32_t rmask;  // and its periodic mask (routes up to 32)
+    int group;       // query heads per KV head
+    int wide;        // staged row strides past RowLoader's 32-bit offsets
 };
 
 // Routing slot of a key: the position of its exponent among the 32 a lane
@@ -596,6 +598,262 @@ flash_bwd_dkdv_kernel(AttnBwdParams p) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// dK/dV of large grids at head_dim 128: 256 keys per block, 32 keys of one
+// query head per wave, all products on v_mfma_f32_32x32x16_bf16 (640
+// bytes of LDS a lane for 32 queries by 32 keys, against the 16-key kernel's
+// 1,024, and half its query staging).
+//  * 32-query chunks of Q and dO, and their lse and D, move from memory
+//    straight into rings of four LDS chunks, two ahead, one barrier per chunk;
+//    K lies in registers, V in LDS (the dK^T and dV^T accumulators take 128
+//    VGPRs);
+//  * S = Q K^T and dP = dO V^T: lane (h, key) holds queries 8 (r / 4) + 4 h +
+//    r % 4, the k order of dV^T += dO^T P and dK^T += Q^T dS, whose A fragments
+//    come by transposing loads from the same chunks;
+//  * masked scores (causal, queries past the sequence) leave P and dS as zero
+//    bits in the packed words, in a branch only the diagonal chunks take;
+//  * dS, where the caller keeps it, leaves through the wave's own 32 x 32 LDS
+//    tile in the dQ kernel's fragment order.
+// Rows past the sequence are staged as its last row; keys past it store
+// nothing.  Waves w and w + 4 share a SIMD and take neighbouring key groups,
+// so each SIMD holds one wave with the routed keys of a 64-key tile at route 32.
+// S 4096, 32 query heads over 8, causal, dS kept, against the 16-key kernel:
+// softmax 351 us (384), D2 at 4 of 32 395 (410), softcap D4 495 (511),
+// B3 414 (435).
+// ---------------------------------------------------------------------------
+struct DkdvShape {
+    static constexpr int kWaves = 8, kKeys = 32 * kWaves, kRing = 4;
+    static constexpr int kChunkB = lds_row<128>(32);  // 32 rows of Q or dO
+    static constexpr int kDsStride = 40;              // BF16 elements per row of the dS tile
+};
+
+template <int MODE, int GRAD, int ROUTE>
+__global__ void __launch_bounds__(64 * DkdvShape::kWaves) __attribute__((amdgpu_waves_per_eu(2)))
+flash_bwd_dkdv256_kernel(AttnBwdParams p) {
+    using F = DkdvShape;
+    constexpr bool kSigmoid = attn_is_sigmoid(MODE);
+    constexpr int HD = 128, W = F::kWaves, kRing = F::kRing, kC = HD / 16, kD = HD / 32;
+    constexpr int kLoadRows = RowLoader<HD>::kLoadRows;
+    // Q ring, dO ring, V; lse and D rings; the waves' dS tiles
+    __shared__ __align__(1024) unsigned char smem[2 * kRing * F::kChunkB + lds_row<HD>(F::kKeys)];
+    __shared__ __align__(16) float stat[2][kRing][64];
+    __shared__ __align__(16) uint16_t dstile[W][32 * F::kDsStride];
+    constexpr uint32_t kDO = kRing * F::kChunkB, kV = 2 * kRing * F::kChunkB;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
+    const uint32_t stat0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) float*)&stat[0][0][0];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int h = lane >> 5, c32 = lane & 31;
+    const int seq = (int)p.seq;
+    const int head = blockIdx.x, b = blockIdx.z, kb = blockIdx.y;
+    const int kvh = (int)((uint32_t)head / (uint32_t)p.group);
+    const int kgroup = 2 * (wave & 3) | (wave >> 2);
+    const int key0 = kb * F::kKeys + 32 * kgroup;  // first key of this wave
+    const int key = key0 + c32;                    // this lane's key
+    const float inv_cap = 1.0f / p.cap;
+    const bool poly_key = key_routed<ROUTE>(p, key);
+    const bool wave_poly = __builtin_amdgcn_ballot_w64(poly_key) != 0;
+
+    const uint16_t* qp = p.q + b * p.qs.b + head * p.qs.h;
+    const uint16_t* dop = p.dout + b * p.dos.b + head * p.dos.h;
+    const uint16_t* kp = p.k + b * p.ks.b + kvh * p.ks.h;
+    const uint16_t* vp = p.v + b * p.vs.b + kvh * p.vs.h;
+    const int64_t statrow = ((int64_t)b * p.hq + head) * p.seq;
+
+    // 32-query chunks, from the block's first key on under the causal mask
+    const int c0 = p.causal ? kb * F::kKeys / 32 : 0;
+    const int nch = (seq + 31) / 32 - c0;
+
+    const RowLoader<HD> loader(lane, p.wide);
+    const TileReader<HD> reader(lane);
+    constexpr int kLoads = 2 * 32 / kLoadRows, kPer = kLoads / W;  // per chunk, and per wave
+    auto load_chunk = [&](int c) {
+        const int slot = c & (kRing - 1);
+        const int q0 = (c0 + c) * 32;
+#pragma unroll
+        for (int j = 0; j < kPer; ++j) {
+            const int n = j * W + wave;
+            const bool second = n >= kLoads / 2;
+            const int r = (n % (kLoads / 2)) * kLoadRows;
+            loader.load(lds0 + (second ? kDO : 0) + slot * F::kChunkB + lds_row<HD>(r), r, second ? dop : qp,
+                        second ? p.dos.s : p.qs.s, q0 + r, seq - 1);
+        }
+        if constexpr (!kSigmoid) {
+            // every wave counts the same loads: even waves move lse, odd ones
+            // D (32 values, twice over; the waves write the same ones)
+            int row = q0 + c32;
+            row = row < seq ? row : seq - 1;
+            const float* src = ((wave & 1) ? p.delta : p.lse) + statrow + row;
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(
+                             __builtin_amdgcn_readfirstlane((int)(stat0 + ((wave & 1) * kRing + slot) * 256))),
+                         "v"(src)
+                         : "memory");
+        }
+    };
+    constexpr int kInFlight = kPer + (kSigmoid ? 0 : 1);
+
+#pragma unroll
+    for (int j = 0; j < 32 / kLoadRows; ++j) {
+        const int r = kLoadRows * (j * W + wave);
+        loader.load(lds0 + kV + lds_row<HD>(r), kLoadRows * wave, vp, p.vs.s, kb * F::kKeys + r, seq - 1);
+    }
+    load_chunk(0);
+    if (nch > 1) load_chunk(1);
+    const int64_t ksrc = key < seq ? key : seq - 1;  // dK and dV of keys past the sequence are not stored
+    bf16x8_t kf[kC];
+#pragma unroll
+    for (int c = 0; c < kC; ++c) kf[c] = *reinterpret_cast<const bf16x8_t*>(kp + ksrc * p.ks.s + c * 16 + h * 8);
+    f32x16_t dk[kD], dv[kD];
+#pragma unroll
+    for (int dt = 0; dt < kD; ++dt) dk[dt] = dv[dt] = (f32x16_t){};
+    const unsigned char* vrows = smem + kV + lds_row<HD>(32 * kgroup);
+
+    auto chunk = [&](int c) {
+        const int slot = c & (kRing - 1);
+        const int q0 = (c0 + c) * 32;
+        const unsigned char* qrows = smem + slot * F::kChunkB;
+        const unsigned char* dorows = smem + kDO + slot * F::kChunkB;
+        __builtin_amdgcn_sched_barrier(0);
+        f32x16_t s = {}, dp = {};
+#pragma unroll
+        for (int i = 0; i < kC; ++i) {
+            s = mfma32(reader.row_frag(qrows, i), kf[i], s);
+            dp = mfma32(reader.row_frag(dorows, i), reader.row_frag(vrows, i), dp);
+        }
+        // three reads per two products, six reads ahead
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+        for (int g = 0; g < 2 * kC; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // register r: query q0 + 8 (r / 4) + 4 h + r % 4 of this lane's key
+        u32x4_t pw[2], sw[2];  // BF16 pairs of P and dS, the B operands of dV and dK
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float lse[4] = {}, del[4] = {};
+            if constexpr (!kSigmoid) {
+                const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&stat[0][slot][8 * g + 4 * h]);
+                const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&stat[1][slot][8 * g + 4 * h]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    lse[r] = l4[r] * kLog2e;
+                    del[r] = d4[r];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const int e = 4 * g + r;
+                float p0, p1, d0, d1;
+                score_grad2<MODE, GRAD, ROUTE>(p, inv_cap, s[e], s[e + 1], dp[e], dp[e + 1], lse[r], lse[r + 1],
+                                               del[r], del[r + 1], poly_key, wave_poly, p0, p1, d0, d1);
+                pw[g >> 1][2 * (g & 1) + (r >> 1)] = pack_bf(p0, p1);
+                sw[g >> 1][2 * (g & 1) + (r >> 1)] = pack_bf(d0, d1);
+            }
+        }
+        if ((p.causal && q0 < key0 + 31) || q0 + 32 > seq) {
+            // the query of row 8 g + r is masked when row < lo or row >= qend
+            const int lo = p.causal ? key - q0 - 4 * h : -64, qend = seq - q0 - 4 * h;
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) {
+                const int row = 8 * (e >> 2) + (e & 3);
+                const uint32_t keep = (row >= lo && row < qend ? 0xffffu : 0u) |
+                                      (row + 1 >= lo && row + 1 < qend ? 0xffff0000u : 0u);
+                pw[e >> 3][(e >> 1) & 3] &= keep;
+                sw[e >> 3][(e >> 1) & 3] &= keep;
+            }
+        }
+        if (p.ds != nullptr) {
+            // as in the 16-key kernel, two 16-key groups at a time; LDS
+            // accesses of one wave complete in order
+            uint16_t* xt = dstile[wave];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const u32x4_t w4 = sw[g >> 1];
+                *reinterpret_cast<u32x2_t*>(xt + c32 * F::kDsStride + 8 * g + 4 * h) =
+                    (g & 1) ? (u32x2_t){w4.z, w4.w} : (u32x2_t){w4.x, w4.y};
+            }
+            __builtin_amdgcn_wave_barrier();
+            const uint16_t* rs = xt + (4 * h + ((lane & 15) >> 2)) * F::kDsStride + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+            u32x2_t dsr[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) dsr[g] = __builtin_bit_cast(u32x2_t, lds_read_tr16(rs + 8 * g * F::kDsStride));
+            __builtin_amdgcn_wave_barrier();
+            const int64_t ch = ds_chunk(b, p.hq, head, p.seq, q0 / 32, key0 / 16);
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+                __builtin_nontemporal_store((u32x4_t){dsr[2 * g].x, dsr[2 * g].y, dsr[2 * g + 1].x, dsr[2 * g + 1].y},
+                                            reinterpret_cast<u32x4_t*>(p.ds) + (ch + g) * 64 + lane);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int dt = 0; dt < kD; ++dt) {
+                dv[dt] = mfma32(reader.col_frag(dorows + lds_row<HD>(16 * g), dt), __builtin_bit_cast(bf16x8_t, pw[g]), dv[dt]);
+                dk[dt] = mfma32(reader.col_frag(qrows + lds_row<HD>(16 * g), dt), __builtin_bit_cast(bf16x8_t, sw[g]), dk[dt]);
+            }
+        __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+        for (int g = 0; g < 4 * kD - 3; ++g) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // sync(c): chunk c has landed for every wave, and every wave is done with
+    // chunk c - 1; loads chunk c + 2.  Still in flight may be the loads of
+    // chunk c + 1 and the two dS stores issued behind them.
+    bool stored = false;
+    auto sync = [&](int c) {
+        if (c + 1 >= nch) wait_loads<0>();
+        else if (stored) wait_loads<kInFlight + 2>();
+        else wait_loads<kInFlight>();
+        block_barrier();
+        if (c + 2 < nch) load_chunk(c + 2);
+    };
+    __builtin_amdgcn_s_waitcnt(0);  // V, K and the first chunks
+    for (int c = 0; c < nch; ++c) {
+        sync(c);
+        const int q0 = (c0 + c) * 32;
+        const bool work = key0 < seq && (!p.causal || q0 + 31 >= key0);
+        if (work) chunk(c);
+        stored = work && p.ds != nullptr;
+    }
+    if (key >= seq) return;
+    // dk[dt][r], dv[dt][r]: head-dim element 32 dt + 8 (r / 4) + 4 h + r % 4 of the lane's key
+    if (p.dkv_ws != nullptr) {
+        const int64_t plane = p.hq * p.seq * HD * (int64_t)gridDim.z;
+        float* wk = p.dkv_ws + ((b * p.hq + head) * p.seq + key) * HD;
+        float* wv = wk + plane;
+#pragma unroll
+        for (int dt = 0; dt < kD; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int d = dt * 32 + 8 * g + 4 * h;
+                *reinterpret_cast<f32x4_t*>(wk + d) = (f32x4_t){dk[dt][4 * g], dk[dt][4 * g + 1], dk[dt][4 * g + 2], dk[dt][4 * g + 3]};
+                *reinterpret_cast<f32x4_t*>(wv + d) = (f32x4_t){dv[dt][4 * g], dv[dt][4 * g + 1], dv[dt][4 * g + 2], dv[dt][4 * g + 3]};
+            }
+        return;
+    }
+    uint16_t* dkr = p.dk + b * p.dks.b + kvh * p.dks.h + key * p.dks.s;
+    uint16_t* dvr = p.dv + b * p.dvs.b + kvh * p.dvs.h + key * p.dvs.s;
+#pragma unroll
+    for (int dt = 0; dt < kD; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int d = dt * 32 + 8 * g + 4 * h;
+            *reinterpret_cast<u32x2_t*>(dkr + d) =
+                (u32x2_t){pack_bf(dk[dt][4 * g], dk[dt][4 * g + 1]), pack_bf(dk[dt][4 * g + 2], dk[dt][4 * g + 3])};
+            *reinterpret_cast<u32x2_t*>(dvr + d) =
+                (u32x2_t){pack_bf(dv[dt][4 * g], dv[dt][4 * g + 1]), pack_bf(dv[dt][4 * g + 2], dv[dt][4 * g + 3])};
+        }
+}
+
 // dK, dV of grouped heads: the sum over the group's query heads of the FP32
 // partials, rounded once to BF16.  Thread = 8 head-dim elements of one key.
 template <int HD>
@@ -937,6 +1195,23 @@ using namespace pt;
 
 namespace {
 
+// Whether the head_dim-128 dK/dV runs 256-key blocks.  One of them a CU does
+// the work of two 128-key blocks in 0.9 of their time, so it pays where its
+// larger grains still fill the rounds.  Causal (heaviest blocks first, 32
+// heads; 128-key against 256-key blocks, softmax / softcap D4): two rounds
+// and more (S 4096, 382 / 522 against 350 / 490 us), at one and a half the
+// softcap loses (S 3072, 242 / 328 against 232 / 345) and at one both (S 2048,
+// 119 / 159 against 140 / 221).  Without the mask all blocks are alike and
+// whole rounds of both count (one round of 256-key blocks, S 2048: 209 against
+// 187; half a round, S 1000: 53 against 70).
+bool dkdv_wide_blocks(const AttnBwdParams& prm, int64_t batch) {
+    const int64_t cus = device_shape().cus, heads = batch * prm.hq;
+    const int64_t blocks = heads * ((prm.seq + DkdvShape::kKeys - 1) / DkdvShape::kKeys);
+    if (prm.causal) return blocks >= 2 * cus;
+    const int64_t rounds = (blocks + cus - 1) / cus, rounds128 = (heads * ((prm.seq + 127) / 128) + cus - 1) / cus;
+    return 19 * rounds <= 10 * rounds128;
+}
+
 template <int MODE, int GRAD, int ROUTE, int HD, bool RAGGED>
 void launch_bwd_shape(const AttnBwdParams& prm, int64_t batch, hipStream_t st) {
     const dim3 grid((unsigned)prm.hq, (unsigned)((prm.seq + 127) / 128), (unsigned)batch);
@@ -948,7 +1223,12 @@ void launch_bwd_shape(const AttnBwdParams& prm, int64_t batch, hipStream_t st) {
     // the dS-keeping backward: the launcher passes a workspace only for
     // aligned lengths and the modes bwd_keeps_ds selects
     constexpr bool kKeepsDs = !RAGGED && bwd_keeps_ds(MODE, HD);
-    if (kKeepsDs && prm.ds != nullptr) {
+    if (HD == 128 && dkdv_wide_blocks(prm, batch)) {
+        const dim3 wgrid(kgrid.x, (unsigned)((prm.seq + DkdvShape::kKeys - 1) / DkdvShape::kKeys), kgrid.z);
+        if constexpr (HD == 128)
+            hipLaunchKernelGGL((flash_bwd_dkdv256_kernel<MODE, GRAD, ROUTE>), wgrid, dim3(64 * DkdvShape::kWaves), 0,
+                               st, prm);
+    } else if (kKeepsDs && prm.ds != nullptr) {
         hipLaunchKernelGGL((flash_bwd_dkdv_kernel<MODE, GRAD, ROUTE, HD, kW, false, kKeepsDs>), kgrid, dim3(64 * kW),
                            0, st, prm);
     } else {
@@ -1090,7 +1370,9 @@ int bwd_run(void* dq, void* dk, void* dv, float* delta, float* dkv_workspace, vo
                       (uint16_t*)dv, grouped ? dkv_workspace : nullptr, keep_ds ? (uint16_t*)ds_workspace : nullptr,
                       st[0], st[1], st[2], st[4], st[5], st[6], st[7], q_heads, kv_heads,
                       seq, scale, cap > 0.0f ? cap : 1.0f, sigmoid_bias, causal != 0, exp2_route,
-                      host_route_mask(exp2_route)};
+                      host_route_mask(exp2_route), (int)(q_heads / kv_heads), 0};
+    // staging adds up to 7 rows to a wave's address as a 32-bit byte offset
+    for (int i : {0, 2, 4}) prm.wide |= st[i].s > (int64_t(1) << 27);
     switch (mode) {
         case kAttnSoftmaxNative: launch_bwd<kAttnSoftmaxNative, kGradNatural, 0>(prm, batch, hst, hd); break;
         case kAttnSoftmaxExp2D2: launch_bwd_routed<kAttnSoftmaxExp2D2>(prm, batch, hst, exp2_route, hd); break;

@@ -1,0 +1,62 @@
+"""dK / dV in 256-key blocks (grids of two rounds and more at head_dim 128)
+against the 128- and 64-key blocks that a few of the same heads run in: dS
+is the same to the bit (so is dQ), and the FP32 sums over queries differ in
+order only.  The small grids' results are compared with the float32
+reference by the other backward tests."""
+
+import math
+
+import pytest
+import torch
+
+from attention_reference import M
+from test_gpu_flash_attention_bwd import _inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _grads(ext, t, mode, grad, causal, route):
+    q, k, v, do = t
+    args = (causal, 1 / math.sqrt(128), 30.0, -math.log(q.shape[1]))
+    out, lse = ext.flash_attn_fwd_bf16(q, k, v, M[mode], 12, *args, -1)
+    return ext.flash_attn_bwd_bf16(q, k, v, out, do, lse, M[mode], grad, route, *args)
+
+
+def _agree(got, want):
+    """BF16 roundings of two FP32 sums of the same n terms, n <= 1000: one
+    step of BF16 apart, or n 2^-24 of the terms' sum near zero (here below
+    2^-12 of the largest result)."""
+    a, b = got.float(), want.float()
+    return bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -12 * b.abs().max()).all())
+
+
+# 512 blocks of 256 keys: one key, a wave's last key, the block's middle and
+# end, one key into the second block, dS kept (256) or not
+@pytest.mark.parametrize("mode,grad,route", [("softmax_native", 0, 0), ("softmax_d2", 0, 32), ("softmax_d2", 0, 14),
+                                             ("softcap_d4", 1, 0), ("sigmoid_d3", 0, 0)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("heads,group,seq", [(512, 4, 1), (512, 1, 32), (512, 4, 161), (512, 1, 256), (256, 8, 257),
+                                             (256, 4, 384), (128, 4, 1000)])
+def test_wide_blocks_match_narrow(spline_ops, cuda, mode, grad, route, causal, heads, group, seq):
+    print(f"dkdv {mode} route {route} causal {causal} heads {heads} group {group} seq {seq}", flush=True)
+    t = [x.to(cuda) for x in _inputs(1, heads, heads // group, seq, seq + group)]
+    many = _grads(spline_ops, t, mode, grad, causal, route)
+    few = _grads(spline_ops, [t[0][:, :, -8:], t[1][:, :, -8 // group:], t[2][:, :, -8 // group:], t[3][:, :, -8:]],
+                 mode, grad, causal, route)
+    assert all(torch.isfinite(g).all() for g in many)
+    assert torch.equal(many[0][:, :, -8:], few[0])
+    for a, b in zip(many[1:], few[1:]):
+        assert _agree(a[:, :, -8 // group:], b)
+
+
+def test_wide_blocks_rows_past_32_bit_offsets(spline_ops, cuda):
+    print("dkdv wide rows", flush=True)
+    t = [x.to(cuda) for x in _inputs(1, 512, 512, 9, 5)]
+    want = _grads(spline_ops, t, "softmax_native", 0, True, 0)
+    step = (1 << 27) + 8
+    base = torch.empty(8 * step + 512 * 128, dtype=torch.bfloat16, device=cuda)
+    wide = base.as_strided((1, 9, 512, 128), (9 * step, step, 128, 1))
+    for i in range(4):
+        wide.copy_(t[i])
+        got = _grads(spline_ops, [wide if j == i else x for j, x in enumerate(t)], "softmax_native", 0, True, 0)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), "q k v dout".split()[i]
