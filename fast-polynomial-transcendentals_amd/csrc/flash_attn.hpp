@@ -257,8 +257,10 @@ __device__ __forceinline__ void wait_loads() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// Block barrier without the waits of __syncthreads, which would also wait for
-// the loads in flight: only memory accesses before it stay before it.
-__device__ __forceinline__ void block_barrier() { asm volatile("s_barrier" ::: "memory"); }
+// Block barrier without __syncthreads' wait for the loads in flight.  The
+// wave's own LDS reads have returned: a load issued behind the barrier may
+// overwrite what they read, and the products that take them need not have
+// been scheduled ahead of it.
+__device__ __forceinline__ void block_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 }  // namespace pt
