@@ -824,29 +824,33 @@ flash_bwd_dkdv256_kernel(AttnBwdParams p) {
         if (work) chunk(c);
         stored = work && p.ds != nullptr;
     }
-    if (key >= seq) return;
+    // the lane's place again from the hardware's lane number: kept over the
+    // loop, it spilled in the softcap D4 and B3 kernels
+    const int lane_end = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const int he = lane_end >> 5, key_end = key0 + (lane_end & 31);
+    if (key_end >= seq) return;
     // dk[dt][r], dv[dt][r]: head-dim element 32 dt + 8 (r / 4) + 4 h + r % 4 of the lane's key
     if (p.dkv_ws != nullptr) {
         const int64_t plane = p.hq * p.seq * HD * (int64_t)gridDim.z;
-        float* wk = p.dkv_ws + ((b * p.hq + head) * p.seq + key) * HD;
+        float* wk = p.dkv_ws + ((b * p.hq + head) * p.seq + key_end) * HD;
         float* wv = wk + plane;
 #pragma unroll
         for (int dt = 0; dt < kD; ++dt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                const int d = dt * 32 + 8 * g + 4 * h;
+                const int d = dt * 32 + 8 * g + 4 * he;
                 *reinterpret_cast<f32x4_t*>(wk + d) = (f32x4_t){dk[dt][4 * g], dk[dt][4 * g + 1], dk[dt][4 * g + 2], dk[dt][4 * g + 3]};
                 *reinterpret_cast<f32x4_t*>(wv + d) = (f32x4_t){dv[dt][4 * g], dv[dt][4 * g + 1], dv[dt][4 * g + 2], dv[dt][4 * g + 3]};
             }
         return;
     }
-    uint16_t* dkr = p.dk + b * p.dks.b + kvh * p.dks.h + key * p.dks.s;
-    uint16_t* dvr = p.dv + b * p.dvs.b + kvh * p.dvs.h + key * p.dvs.s;
+    uint16_t* dkr = p.dk + b * p.dks.b + kvh * p.dks.h + key_end * p.dks.s;
+    uint16_t* dvr = p.dv + b * p.dvs.b + kvh * p.dvs.h + key_end * p.dvs.s;
 #pragma unroll
     for (int dt = 0; dt < kD; ++dt)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const int d = dt * 32 + 8 * g + 4 * h;
+            const int d = dt * 32 + 8 * g + 4 * he;
             *reinterpret_cast<u32x2_t*>(dkr + d) =
                 (u32x2_t){pack_bf(dk[dt][4 * g], dk[dt][4 * g + 1]), pack_bf(dk[dt][4 * g + 2], dk[dt][4 * g + 3])};
             *reinterpret_cast<u32x2_t*>(dvr + d) =
