@@ -185,7 +185,18 @@ __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint
                  : "memory");
 }
 
-// The same with an address of each lane's own.
+// The same for memory read once: it does not displace what the caches hold.
+__device__ __forceinline__ void load_to_lds_once(uint32_t lds, const void* base, uint32_t offset) {
+    const uint64_t bits = (uint64_t)(uintptr_t)base;
+    const uint64_t sbase = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(bits >> 32)) << 32) |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bits);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :
+                 : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(offset), "s"(sbase)
+                 : "memory");
+}
+
+// load_to_lds with an address of each lane's own.
 __device__ __forceinline__ void load_to_lds_each(uint32_t lds, const void* lane_src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                  :

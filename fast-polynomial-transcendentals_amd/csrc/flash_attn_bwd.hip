@@ -1084,113 +1084,106 @@ __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))
 // ---------------------------------------------------------------------------
 // dQ from the dS chunks of the dK/dV kernel (the dS-keeping backward):
 // dQ^T += K^T dS^T.  A block of 4 waves owns 128 queries of one query head
-// (32 per wave), streams 64-key tiles of K through LDS (K^T fragments by the
-// transposing loads of frag_tr32) and loads each chunk straight into the B
-// fragment registers.  K is loaded one tile ahead and dS two (a ring of
-// three fragment sets: measured on MI355X 1.02x for the whole head_dim-128
-// backward against one tile ahead, bit-identical); the loop is unrolled by
-// six, so every ring index is static and no register copy waits for a
-// load.  Under the causal mask a wave multiplies the chunks of keys up to
-// its last query, the ones the dK/dV kernel wrote.  S a multiple of 128.
+// (32 per wave).  What bounds it is the stream of dS from memory, so tiles
+// of K and each wave's own chunks of dS move straight into LDS rings, counted
+// in flight together, one barrier per tile (K and dS through registers: the
+// waits for K held back the dS behind it).  64-key tiles one ahead at
+// head_dim 128, 32-key tiles three ahead at 64, two and three blocks per CU.
+// Where the head count allows it, workgroups that share an XCD (every eighth
+// one) take neighbouring heads, which read the same K.  Under the causal mask
+// a wave multiplies the groups of keys up to its last query, the ones the
+// dK/dV kernel wrote.  S a multiple of 128.
+// S 4096, 32 heads over 8, causal, 128 against 64 dimensions: 126 and 108 us
+// (through registers 150 and 129; dS alone takes 84 at the rate of a copy);
+// 32-key tiles three ahead at 128 129 us, 64-key ones at 64 113, 8-wave blocks
+// 133 at best.
 // ---------------------------------------------------------------------------
 template <int HD>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 64 ? 4 : 2)))
+struct DqDsShape {
+    static constexpr int kTile = HD == 128 ? 64 : 32, kRing = HD == 128 ? 2 : 4;
+    static constexpr int kGroups = kTile / 16;  // 16-key groups: 1 KiB of dS per wave each
+    static constexpr int kKB = lds_row<HD>(kTile), kDsB = 4 * kGroups * 1024;
+};
+
+template <int HD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD == 128 ? 2 : 3)))
 flash_bwd_dq_ds_kernel(AttnBwdParams p) {
-    constexpr int kRS = k_row_stride<HD>(), kChunks = HD / 8;
-    constexpr int kKT = 64;                   // keys per staged tile
-    constexpr int kRowsPass = 256 / kChunks;  // K rows one pass of the block moves
-    constexpr int kPasses = kKT / kRowsPass;
-    __shared__ __align__(16) uint16_t ktile[2][kKT * kRS];
+    using F = DqDsShape<HD>;
+    constexpr int kRing = F::kRing, kG = F::kGroups, kLoadRows = RowLoader<HD>::kLoadRows;
+    constexpr int kLoads = F::kTile / kLoadRows / 4;  // of K, per wave and tile
+    static_assert(kLoads * kLoadRows * 4 == F::kTile, "four waves stage a K tile");
+    __shared__ __align__(1024) unsigned char smem[kRing * (F::kKB + F::kDsB)];  // K ring, dS ring
+    constexpr uint32_t kDs = kRing * F::kKB;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem;
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int h = lane >> 5, c32 = lane & 31;
-    const int64_t nqb = p.seq / 128;
-    const int64_t head = blockIdx.x, b = blockIdx.z;
-    const int64_t qb = p.causal ? nqb - 1 - (int64_t)blockIdx.y : (int64_t)blockIdx.y;
-    const int64_t kvh = head / (p.hq / p.hkv);
-    const int64_t q0 = qb * 128 + wave * 32;
-    const int64_t qrow = q0 + c32;
-    const u32x4_t* dsrc = reinterpret_cast<const u32x4_t*>(p.ds) + ds_chunk(b, p.hq, head, p.seq, q0 / 32, 0) * 64 + lane;
-    const int64_t kglim = p.causal ? q0 / 16 + 1 : p.seq / 16 - 1;  // the wave's last 16-key group
+    const int seq = (int)p.seq, hq = (int)p.hq;
+    const int head = hq % 8 == 0 ? (int)(blockIdx.x & 7) * (hq / 8) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+    const int b = blockIdx.z;
+    const int qb = p.causal ? seq / 128 - 1 - (int)blockIdx.y : (int)blockIdx.y;
+    const int kvh = (int)((uint32_t)head / (uint32_t)p.group);
+    const int q0 = qb * 128 + wave * 32;
+    const uint16_t* kp = p.k + b * p.ks.b + kvh * p.ks.h;
+    const unsigned char* dsp =
+        reinterpret_cast<const unsigned char*>(p.ds) + ds_chunk(b, p.hq, head, p.seq, q0 / 32, 0) * 1024;
+    const int ngroups = p.causal ? q0 / 16 + 2 : seq / 16;  // of this wave
+    const int nkt = (p.causal ? (qb + 1) * 128 : seq) / F::kTile;
+
+    const RowLoader<HD> loader(lane, p.wide);
+    const TileReader<HD> reader(lane);
+    // Every 16-key group of the tiles a block walks lies inside the workspace
+    // (group < S / 16); groups past the wave's last hold no dS and are not
+    // multiplied.
+    auto load_tile = [&](int t) {
+        const uint32_t slot = (uint32_t)(t % kRing);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) {
+            const int r = kLoadRows * (j * 4 + wave);
+            loader.load(lds0 + slot * F::kKB + lds_row<HD>(r), kLoadRows * wave, kp, p.ks.s, t * F::kTile + r, seq - 1);
+        }
+#pragma unroll
+        for (int g = 0; g < kG; ++g)
+            load_to_lds_once(lds0 + kDs + slot * F::kDsB + (wave * kG + g) * 1024, dsp + (int64_t)(t * kG + g) * 1024,
+                             lane * 16);
+    };
+    constexpr int kInFlight = (kLoads + kG) * (kRing - 2);
 
     f32x16_t dqacc[HD / 32];
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt) dqacc[dt] = (f32x16_t){};
-
-    const int krow = tid / kChunks, kcol = (tid % kChunks) * 8;
-    const uint16_t* kp = p.k + b * p.ks.b + kvh * p.ks.h + krow * p.ks.s + kcol;
-    u32x4_t kr[kPasses];  // K rows of the next tile
-    u32x4_t dsf[3][4];    // dS fragments of this tile and the next two, by t mod 3
-    const int64_t ktiles = p.seq / kKT;
-    const int64_t ncausal = p.causal ? (qb + 1) * (128 / kKT) : ktiles;
-    const int64_t nkt = ncausal < ktiles ? ncausal : ktiles;
-    const int tr_off = (4 * h + ((lane & 15) >> 2)) * kRS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-
-    auto kload = [&](int64_t t) {
 #pragma unroll
-        for (int j = 0; j < kPasses; ++j)
-            kr[j] = *reinterpret_cast<const u32x4_t*>(kp + (t * kKT + kRowsPass * j) * p.ks.s);
-    };
-    auto kstore = [&](int par) {
+    for (int t = 0; t < kRing - 1; ++t)
+        if (t < nkt) load_tile(t);
+    for (int t = 0; t < nkt; ++t) {
+        // tile t has landed, the kRing - 2 behind it may be in flight; every
+        // wave is done with tile t - 1, whose slot the next load takes
+        if (kRing > 2 && t + kRing - 2 < nkt) wait_loads<kInFlight>();
+        else wait_loads<0>();
+        block_barrier();
+        if (t + kRing - 1 < nkt) load_tile(t + kRing - 1);
+        const unsigned char* krows = smem + t % kRing * F::kKB;
+        const unsigned char* ds = smem + kDs + t % kRing * F::kDsB + wave * kG * 1024 + lane * 16;
 #pragma unroll
-        for (int j = 0; j < kPasses; ++j)
-            *reinterpret_cast<u32x4_t*>(&ktile[par][(krow + kRowsPass * j) * kRS + kcol]) = kr[j];
-    };
-    // Every 16-key group of the tiles a wave walks lies inside the
-    // workspace (group < S / 16); groups past the causal limit hold no dS
-    // and the products skip them.
-    auto dload = [&](int slot, int64_t t) {
+        for (int g = 0; g < kG; ++g) {
+            if (t * kG + g < ngroups) {  // wave-uniform
+                const bf16x8_t sf = *reinterpret_cast<const bf16x8_t*>(ds + g * 1024);
 #pragma unroll
-        for (int cc = 0; cc < 4; ++cc) dsf[slot][cc] = __builtin_nontemporal_load(dsrc + (4 * t + cc) * 64);
-    };
-    // tile t: K in ktile[t % 2], dS in dsf[t % 3]; issue K of t + 1 (staged
-    // after the products) and dS of t + 2
-    auto step = [&](auto kpar_c, auto dslot_c, int64_t t) {
-        constexpr int KP = decltype(kpar_c)::value, DS = decltype(dslot_c)::value;
-        if (t + 1 < nkt) kload(t + 1);
-        if (t + 2 < nkt) dload((DS + 2) % 3, t + 2);
-        if (4 * t <= kglim) {  // wave-uniform
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc) {
-                if (4 * t + cc <= kglim) {
-                    const bf16x8_t sf = __builtin_bit_cast(bf16x8_t, dsf[DS][cc]);
-#pragma unroll
-                    for (int dt = 0; dt < HD / 32; ++dt)
-                        dqacc[dt] = mfma32(frag_tr32<HD>(ktile[KP] + tr_off, dt, cc), sf, dqacc[dt]);
-                }
+                for (int dt = 0; dt < HD / 32; ++dt)
+                    dqacc[dt] = mfma32(reader.col_frag(krows + lds_row<HD>(16 * g), dt), sf, dqacc[dt]);
             }
         }
-        if (t + 1 < nkt) kstore(KP ^ 1);
-        __syncthreads();
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    kload(0);
-    kstore(0);
-    dload(0, 0);
-    if (nkt > 1) dload(1, 1);
-    __syncthreads();
-    for (int64_t t = 0; t < nkt; t += 6) {
-        step(I0{}, I0{}, t);
-        if (t + 1 < nkt) step(I1{}, I1{}, t + 1);
-        if (t + 2 < nkt) step(I0{}, I2{}, t + 2);
-        if (t + 3 < nkt) step(I1{}, I0{}, t + 3);
-        if (t + 4 < nkt) step(I0{}, I1{}, t + 4);
-        if (t + 5 < nkt) step(I1{}, I2{}, t + 5);
     }
 
-    uint16_t* dqr = p.dq + b * p.dqs.b + head * p.dqs.h + qrow * p.dqs.s;
+    uint16_t* dqr = p.dq + b * p.dqs.b + head * p.dqs.h + (q0 + c32) * p.dqs.s;
 #pragma unroll
     for (int dt = 0; dt < HD / 32; ++dt)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int d = dt * 32 + 8 * g + 4 * h;
-            const u32x2_t w = {pack_bf(dqacc[dt][4 * g], dqacc[dt][4 * g + 1]),
-                               pack_bf(dqacc[dt][4 * g + 2], dqacc[dt][4 * g + 3])};
-            *reinterpret_cast<u32x2_t*>(dqr + d) = w;
-        }
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<u32x2_t*>(dqr + dt * 32 + 8 * g + 4 * h) =
+                (u32x2_t){pack_bf(dqacc[dt][4 * g], dqacc[dt][4 * g + 1]),
+                          pack_bf(dqacc[dt][4 * g + 2], dqacc[dt][4 * g + 3])};
 }
 
 }  // namespace pt
@@ -1376,7 +1369,7 @@ int bwd_run(void* dq, void* dk, void* dv, float* delta, float* dkv_workspace, vo
                       seq, scale, cap > 0.0f ? cap : 1.0f, sigmoid_bias, causal != 0, exp2_route,
                       host_route_mask(exp2_route), (int)(q_heads / kv_heads), 0};
     // staging adds up to 7 rows to a wave's address as a 32-bit byte offset
-    for (int i : {0, 2, 4}) prm.wide |= st[i].s > (int64_t(1) << 27);
+    for (int i : {0, 1, 2, 4}) prm.wide |= st[i].s > (int64_t(1) << 27);
     switch (mode) {
         case kAttnSoftmaxNative: launch_bwd<kAttnSoftmaxNative, kGradNatural, 0>(prm, batch, hst, hd); break;
         case kAttnSoftmaxExp2D2: launch_bwd_routed<kAttnSoftmaxExp2D2>(prm, batch, hst, exp2_route, hd); break;

@@ -60,3 +60,19 @@ def test_wide_blocks_rows_past_32_bit_offsets(spline_ops, cuda):
         wide.copy_(t[i])
         got = _grads(spline_ops, [wide if j == i else x for j, x in enumerate(t)], "softmax_native", 0, True, 0)
         assert all(torch.equal(a, b) for a, b in zip(got, want)), "q k v dout".split()[i]
+
+
+# dQ from the kept dS: heads in eighths (mapped by XCD) or not, one tile to
+# several rings of them
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("heads,group,seq", [(2, 1, 128), (8, 4, 256), (12, 4, 384), (24, 3, 128), (16, 2, 640)])
+def test_dq_from_ds_matches_recomputed(spline_ops, cuda, monkeypatch, d, causal, heads, group, seq):
+    print(f"dq d {d} causal {causal} heads {heads} group {group} seq {seq}", flush=True)
+    q, k, v, do = (x.to(cuda) for x in _inputs(2, heads, heads // group, seq, seq + d, qmul=6.0, d=d))
+    args = (causal, 1 / math.sqrt(d), 30.0, 0.0)
+    out, lse = spline_ops.flash_attn_fwd_bf16(q, k, v, M["softcap_d4"], 4, *args, -1)
+    got = spline_ops.flash_attn_bwd_bf16(q, k, v, out, do, lse, M["softcap_d4"], 1, 0, *args)
+    monkeypatch.setenv("SPLINE_ATTN_DS_MAX_BYTES", "0")
+    want = spline_ops.flash_attn_bwd_bf16(q, k, v, out, do, lse, M["softcap_d4"], 1, 0, *args)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
