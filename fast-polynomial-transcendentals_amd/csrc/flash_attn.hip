@@ -307,10 +307,9 @@ constexpr int fwd_waves_per_eu() {
 // and the head index varies fastest, so the first wave of resident blocks
 // takes the longest query blocks of every head.
 //
-// Any S: rows past the last real key are staged as that key's row (a finite
-// row times a masked probability, which is 0), queries past the sequence
-// compute the last query's row and store nothing, and a wave with no query
-// at all only stages.
+// Any S: rows past the last real key are staged as zeros (their probability
+// is 0), queries past the sequence take a row of zeros and store nothing, and
+// a wave with no query at all only stages.
 template <int MODE, int ROUTE, int HD, int W>
 __global__ void __launch_bounds__(64 * W)
     __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu<MODE, HD>()))) flash_fwd_kernel(AttnParams p) {

@@ -204,6 +204,9 @@ __device__ __forceinline__ void load_to_lds_each(uint32_t lds, const void* lane_
                  : "memory");
 }
 
+// What rows past the end are loaded from.
+static __device__ const uint32_t kZeroChunk[4] __attribute__((aligned(16))) = {0u, 0u, 0u, 0u};
+
 // Stages rows of HD BF16 values, kLoadRows per load; wave and rows of a load as
 // the kernel divides them, in whole multiples of kLoadRows.
 template <int HD>
@@ -217,15 +220,16 @@ struct RowLoader {
 
     // Rows row0 .. row0 + kLoadRows - 1 of base to LDS address lds (their
     // lds_row in some tile, tile_row = row0's row there modulo 8).  Rows past
-    // `last` read it.
+    // `last` are zeros: a copy of a real row that holds an infinity would meet
+    // the zero probability of a masked one, and 0 * Inf is NaN.
     __device__ __forceinline__ void load(uint32_t lds, int tile_row, const uint16_t* base, int64_t stride, int row0,
                                          int last) const {
         const uint32_t col = (uint32_t)((lc ^ row_swizzle<HD>(tile_row + lr)) * 16);
         if (row0 + kLoadRows - 1 <= last && !wide) {  // wave-uniform
             load_to_lds(lds, base + row0 * stride, (uint32_t)lr * (uint32_t)(int)stride * 2 + col);
         } else {
-            const int row = row0 + lr < last ? row0 + lr : last;
-            load_to_lds_each(lds, reinterpret_cast<const unsigned char*>(base + row * stride) + col);
+            const unsigned char* src = reinterpret_cast<const unsigned char*>(base + (row0 + lr) * stride) + col;
+            load_to_lds_each(lds, row0 + lr <= last ? src : reinterpret_cast<const unsigned char*>(kZeroChunk));
         }
     }
 };

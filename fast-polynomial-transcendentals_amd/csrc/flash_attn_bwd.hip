@@ -614,7 +614,7 @@ flash_bwd_dkdv_kernel(AttnBwdParams p) {
 //    bits in the packed words, in a branch only the diagonal chunks take;
 //  * dS, where the caller keeps it, leaves through the wave's own 32 x 32 LDS
 //    tile in the dQ kernel's fragment order.
-// Rows past the sequence are staged as its last row; keys past it store
+// Rows past the sequence are staged as zeros; keys past it store
 // nothing.  Waves w and w + 4 share a SIMD and take neighbouring key groups,
 // so each SIMD holds one wave with the routed keys of a 64-key tile at route 32.
 // S 4096, 32 query heads over 8, causal, dS kept, against the 16-key kernel:

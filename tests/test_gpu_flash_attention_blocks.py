@@ -99,3 +99,17 @@ def test_wrapper_output_and_gradient_layouts(cuda, own):
                            ("expanded", grads(row), grads(row.contiguous())),
                            ("edited", grads(do / 2, edit=True), want)):  # halves and doubles are exact
         assert all(torch.equal(a, b) for a, b in zip(got, ref)), name
+
+
+# rows past the last key reach the products with probability 0: they hold
+# zeros, not a copy of a row whose infinity would make them NaN.  4- and
+# 8-wave blocks, a tile's first, middle and last row
+@pytest.mark.parametrize("mode", ["softmax_native", "softcap_native", "sigmoid_native"])
+@pytest.mark.parametrize("d,heads,seq", [(64, 4, 65), (64, 4, 200), (128, 4, 127), (128, 512, 33)])
+def test_infinite_last_row_of_v(spline_ops, cuda, mode, d, heads, seq):
+    print(f"infinite v {mode} d {d} heads {heads} seq {seq}", flush=True)
+    q, k, v = (t.to(cuda) for t in _inputs(1, heads, heads, seq, d + seq, d=d)[:3])
+    v[:, -1, :, 3] = float("inf")
+    out = spline_ops.flash_attn_fwd_bf16(q, k, v, M[mode], 12, False, 1 / math.sqrt(d), 30.0, 0.0, -1)[0]
+    assert (out[..., 3] == float("inf")).all()
+    assert torch.isfinite(out[..., :3]).all() and torch.isfinite(out[..., 4:]).all()

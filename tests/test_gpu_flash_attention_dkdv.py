@@ -76,3 +76,16 @@ def test_dq_from_ds_matches_recomputed(spline_ops, cuda, monkeypatch, d, causal,
     monkeypatch.setenv("SPLINE_ATTN_DS_MAX_BYTES", "0")
     want = spline_ops.flash_attn_bwd_bf16(q, k, v, out, do, lse, M["softcap_d4"], 1, 0, *args)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("mode", ["softmax_native", "sigmoid_native"])
+@pytest.mark.parametrize("heads", [512, 8])  # 256-key blocks, and smaller ones
+def test_infinite_last_row_of_dout(spline_ops, cuda, mode, heads):
+    """Queries past the sequence add zeros to dV, not a masked probability
+    times the last row's infinity."""
+    print(f"infinite dout {mode} heads {heads}", flush=True)
+    t = [x.to(cuda) for x in _inputs(1, heads, heads, 161, 161)]
+    t[3][:, -1, :, 3] = float("inf")
+    dv = _grads(spline_ops, t, mode, 0, False, 0)[2]
+    assert (dv[..., 3] == float("inf")).all()
+    assert torch.isfinite(dv[..., :3]).all() and torch.isfinite(dv[..., 4:]).all()
