@@ -174,12 +174,18 @@ template <int HD>
 __device__ __forceinline__ constexpr uint32_t lds_row(int row) { return (uint32_t)(row * HD * 2 + (row >> 3) * 32); }
 
 // Moves lane 16 bytes of memory at base + offset (bytes) to LDS address lds +
-// 16 * lane; lds and base wave-uniform.
+// 16 * lane; lds and base wave-uniform.  The compiler does not look into the
+// asm for wait states: an SGPR that a vector instruction wrote (the
+// v_readfirstlane of base, or the v_readlane of a spilled one) may be read as
+// an address five wait states later, M0 one after it was written.
+// s_mov_b32 and s_nop 3 are five.  M0 is reserved: the compiler puts no value
+// there but for an instruction that reads it, and these kernels have none
+// outside the asm (a clobber of a reserved register means nothing to it).
 __device__ __forceinline__ void load_to_lds(uint32_t lds, const void* base, uint32_t offset) {
     const uint64_t bits = (uint64_t)(uintptr_t)base;
     const uint64_t sbase = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(bits >> 32)) << 32) |
                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bits);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
                  : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(offset), "s"(sbase)
                  : "memory");
@@ -190,13 +196,14 @@ __device__ __forceinline__ void load_to_lds_once(uint32_t lds, const void* base,
     const uint64_t bits = (uint64_t)(uintptr_t)base;
     const uint64_t sbase = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(bits >> 32)) << 32) |
                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)bits);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2 nt"
                  :
                  : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(offset), "s"(sbase)
                  : "memory");
 }
 
-// load_to_lds with an address of each lane's own.
+// load_to_lds with an address of each lane's own, in VGPRs (no wait states but
+// M0's).
 __device__ __forceinline__ void load_to_lds_each(uint32_t lds, const void* lane_src) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                  :

@@ -16,7 +16,9 @@ its name carries:
 * no kernel issues packed FP32 arithmetic (v_pk_fma_f32, v_pk_mul_f32,
   v_pk_add_f32): the build turns the packed-fp32-ops target feature off;
 * no kernel spills registers to scratch memory (the code objects' AMDGPU
-  metadata), apart from one measured exception.
+  metadata), apart from one measured exception;
+* every load from memory to LDS has its wait states: M0 written ahead of it,
+  and five behind a vector instruction that wrote its scalar address.
 
 Runs on the CPU (no GPU, no compute)."""
 
@@ -100,28 +102,91 @@ def metadata():
     return [(re.sub(r"\(.*", "", d), spill, scratch) for d, (_, spill, scratch) in zip(demangled, rows)]
 
 
+LDS_LOAD = re.compile(r"^(global|buffer|scratch)_load_lds_|^buffer_load_\w+ .*\blds\b")
+SGPRS = re.compile(r"\bs\[(\d+):(\d+)\]|\bs(\d+)\b|\bvcc\b")
+TWO_RESULTS = re.compile(r"^v_(\w*_co_\w+|div_scale_\w+|mad_[ui]64_\w+)$")  # a scalar one behind the vector one
+
+
+def _sgprs(operands: str) -> set:
+    out = set()
+    for m in SGPRS.finditer(operands):
+        if m.group(1):
+            out.update(range(int(m.group(1)), int(m.group(2)) + 1))
+        else:
+            out.add(int(m.group(3)) if m.group(3) else "vcc")
+    return out
+
+
+def _wait_state_faults(window: list, load: str) -> list:
+    """What a load to LDS breaks, from the instructions ahead of it (nearest
+    last; a branch target between them would only add wait states)."""
+    address = _sgprs(load.split(None, 1)[1])
+    faults, states, m0_seen = [], 0, False
+    for line in reversed(window):
+        op, _, rest = line.partition(" ")
+        operands = rest.split(",")
+        if states < 1 and operands[0].strip() == "m0":
+            faults.append(f"M0 written {states} wait states ahead of: {load}")
+        m0_seen = m0_seen or operands[0].strip() == "m0"
+        if states < 5 and op.startswith("v_"):
+            written = _sgprs(operands[0]) | (_sgprs(operands[1]) if TWO_RESULTS.match(op) else set())
+            if written & address:
+                faults.append(f"{line} {states} wait states ahead of: {load}")
+        states += int(rest.split()[0]) + 1 if op == "s_nop" else 1
+    return faults if m0_seen else faults + [f"no write of M0 ahead of: {load}"]
+
+
+def test_wait_state_audit_counts():
+    """The rules of _wait_state_faults on written-out sequences."""
+    load = "global_load_lds_dwordx4 v6, s[34:35]"
+    base, m0 = "v_readfirstlane_b32 s34, v1", "s_mov_b32 m0, s20"
+    assert _wait_state_faults([base, m0, "s_nop 0"], load)
+    assert _wait_state_faults([base, m0, "s_nop 2"], load)
+    assert not _wait_state_faults([base, m0, "s_nop 3"], load)
+    assert not _wait_state_faults(["v_readfirstlane_b32 s36, v1", m0, "s_nop 0"], load)
+    assert _wait_state_faults(["v_add_co_u32_e64 v0, s[34:35], v1, v2", m0, "s_nop 0"], load)
+    assert not _wait_state_faults(["v_add_f32_e32 v0, s34, v2", m0, "s_nop 0"], load)
+    assert _wait_state_faults([m0], load) and _wait_state_faults(["s_nop 4"], load)
+
+
 @pytest.fixture(scope="module")
-def kernels():
-    """Demangled kernel name (without parameters) -> Counter of mnemonics."""
+def disassembly():
+    """Demangled kernel name (without parameters) -> Counter of mnemonics, and
+    -> [loads to LDS, the wait states that they lack, instructions that name
+    M0]."""
     if not os.path.exists(OBJDUMP) or not os.path.exists(OBJCOPY):
         pytest.skip("ROCm llvm-objdump / llvm-objcopy not found")
     assert os.path.exists(capi_helpers.LIB), "build the library first (__graft_entry__.build())"
     out = collections.defaultdict(collections.Counter)
+    lds_loads = collections.defaultdict(lambda: [0, [], 0])
     with tempfile.TemporaryDirectory() as tmp:
         objects = _code_objects(capi_helpers.LIB, tmp)
         assert objects, "no gfx950 code object in the library"
         for obj in objects:
             text = subprocess.run([OBJDUMP, "-d", "-C", "--no-show-raw-insn", "--no-leading-addr", obj],
                                   check=True, capture_output=True, text=True).stdout
-            name = None
+            name, window = None, collections.deque(maxlen=8)
             for line in text.splitlines():
                 m = re.match(r"^<(.+)>:$", line)
                 if m:
                     name = re.sub(r"\(.*", "", m.group(1))
+                    window.clear()
                     continue
                 if name and line.startswith("\t"):
                     out[name][line.split()[0]] += 1
-    return out
+                    instruction = line.split("//")[0].strip()
+                    if re.search(r"\bm0\b", instruction):
+                        lds_loads[name][2] += 1
+                    if LDS_LOAD.match(instruction):
+                        lds_loads[name][0] += 1
+                        lds_loads[name][1] += _wait_state_faults(list(window), instruction)
+                    window.append(instruction)
+    return out, lds_loads
+
+
+@pytest.fixture(scope="module")
+def kernels(disassembly):
+    return disassembly[0]
 
 
 def _uses(counter, pattern) -> list:
@@ -172,6 +237,21 @@ def test_polynomial_kernels_issue_no_transcendental(kernels):
         if hits:
             bad[name] = hits
     assert not bad, bad
+
+
+def test_loads_to_lds_have_their_wait_states(disassembly):
+    """An SGPR written by a vector instruction (v_readfirstlane of an address,
+    v_readlane of a spilled one) may be read as an address five wait states
+    later, and M0 one wait state after it was written.  The compiler pads its
+    own loads so; what inline assembly holds it does not see.  Nothing but
+    these loads uses M0, which they overwrite."""
+    _, lds_loads = disassembly
+    for family in ("flash_fwd_kernel", "flash_bwd_dkdv256_kernel", "flash_bwd_dq_ds_kernel"):
+        assert any(f"pt::{family}<" in k and n for k, (n, _, _) in lds_loads.items()), family
+    bad = {k: faults[:2] for k, (_, faults, _) in lds_loads.items() if faults}
+    assert not bad, (len(bad), list(bad.items())[:3])
+    others = {k: (n, m0) for k, (n, _, m0) in lds_loads.items() if n and m0 != n}
+    assert not others, list(others.items())[:3]
 
 
 @pytest.mark.parametrize("pattern,needed", [
