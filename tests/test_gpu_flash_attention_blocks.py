@@ -66,6 +66,26 @@ def test_heads_first_output(spline_ops, cuda, mode, d, heads, seq):
     assert torch.equal(kept, out) and torch.equal(kept_lse, lse)
 
 
+@pytest.mark.parametrize("heads,seq", [(4, 130), (1, 130), (1, 1)])
+def test_misaligned_gradient_layouts(cuda, heads, seq):
+    """A gradient whose transposed view is contiguous at an address or at
+    strides that 16-byte loads cannot take is copied."""
+    from sfu_repro.fa4 import FA4Config, build_fa4_module
+
+    print(f"misaligned gradient heads {heads} seq {seq}", flush=True)
+    module = build_fa4_module(FA4Config(), head_dim=64)
+    q, k, v, do = (t.transpose(1, 2).contiguous().to(cuda) for t in _inputs(2, heads, heads, seq, 7, d=64))
+    leaves = [t.clone().requires_grad_() for t in (q, k, v)]
+    out = module(*leaves)
+    want = torch.autograd.grad(out, leaves, do, retain_graph=True)
+    memory = torch.empty(do.numel() + 1, dtype=do.dtype, device=cuda)[1:]
+    for shape in ((2, heads, seq, 64), (2, seq, heads, 64)):
+        dout = memory.view(shape)
+        dout = (dout if shape[1] == heads else dout.transpose(1, 2)).copy_(do)
+        got = torch.autograd.grad(out, leaves, dout, retain_graph=True)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), shape
+
+
 @pytest.mark.parametrize("own", [True, False])
 def test_wrapper_output_and_gradient_layouts(cuda, own):
     """The module's output is contiguous and the caller's to edit, and the
