@@ -116,7 +116,10 @@ packed_bwd_kernel(const void* __restrict__ grad_out, const void* __restrict__ pa
     }
 }
 
-// Element path (odd H or H < 8, storage not 4-byte aligned, or >= 2^31 vectors).
+// Element path (odd H or H < 8, storage not 4-byte aligned, >= 2^31 vectors, or
+// gradients over the rows that they are the gradients of at an H whose vectors
+// overlap: the second of two overlapping vectors would read what the first
+// stored).
 template <class Op, bool BWD>
 __global__ void __launch_bounds__(kBlock)
 packed_element_kernel(const void* __restrict__ grad_out, const void* __restrict__ packed,
@@ -151,8 +154,12 @@ int launch_packed(void* out, const void* grad_out, const void* packed, int64_t r
     if (n == 0) return hipSuccess;
     if (!out || !packed || (BWD && !grad_out)) return hipErrorInvalidValue;
     const auto aligned4 = [](const void* p) { return ((uintptr_t)p & 3u) == 0; };
+    const auto apart = [out, out_bytes = (BWD ? 4 : 2) * n](const void* in, int64_t bytes) {
+        return (uintptr_t)out + out_bytes <= (uintptr_t)in || (uintptr_t)in + bytes <= (uintptr_t)out;
+    };
+    const bool once = h % 8 == 0 || (apart(packed, 4 * n) && (!BWD || apart(grad_out, 2 * n)));
     const int64_t nv = (h + 7) / 8, n_vec = rows * nv;
-    const bool vec = h % 2 == 0 && h >= 8 && aligned4(out) && aligned4(packed) && (!BWD || aligned4(grad_out)) &&
+    const bool vec = h % 2 == 0 && h >= 8 && once && aligned4(out) && aligned4(packed) && (!BWD || aligned4(grad_out)) &&
                      n_vec < (int64_t(1) << 31) && h < (int64_t(1) << 31);
     if (!vec) {
         const int64_t grid = grid_one_pass(n);

@@ -182,6 +182,21 @@ def test_packed_rows_of_any_width(capi, cuda, rows, hidden, offset):
         assert bool((whole[:guard + offset] == 7).all()) and bool((whole[guard + offset + count:] == 7).all())
 
 
+@pytest.mark.parametrize("hidden", [8, 9, 14, 2730])
+def test_packed_gradients_over_their_inputs(capi, cuda, hidden):
+    """grad_packed written over packed, at widths whose row vectors overlap
+    and at ones where they do not."""
+    rows = 65
+    torch.manual_seed(hidden)
+    packed = (torch.randn(rows, 2 * hidden, device=cuda) * 3).to(torch.bfloat16)
+    go = torch.randn(rows, hidden, device=cuda).to(torch.bfloat16)
+    want = torch.empty_like(packed)
+    capi.call("launch_swish_mul_packed_bwd_d3_kernel_bf16", want, go, packed, rows, hidden)
+    capi.call("launch_swish_mul_packed_bwd_d3_kernel_bf16", packed, go, packed, rows, hidden)
+    torch.cuda.synchronize()
+    assert torch.equal(packed.view(torch.int16), want.view(torch.int16))
+
+
 def test_b3_exhaustive(capi, oracle, cuda):
     x = oracle.all_bits()
     xd = _dev(x, "bf16", cuda)
