@@ -20,7 +20,15 @@ def _out(ext, q, k, v, mode, causal, valid=-1):
     return (out, lse) if lse.any() else (out,)
 
 
-# one round of 512 blocks of 256 queries: 1, 2 and 4 blocks a head, their
+def _eight_waves(heads, seq):
+    """The launcher's rule for 8-wave blocks at head_dim 128 (fwd_waves in
+    flash_attn.hip), which has to change with it."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = heads * -(-seq // 256)
+    return blocks % (2 * cus) == 0 or blocks >= 10 * cus
+
+
+# two rounds of 256 blocks of 256 queries: 1, 2 and 4 blocks a head, their
 # last ones full, one query, and ending inside a tile or a wave
 @pytest.mark.parametrize("mode", ["softmax_native", "softcap_d4", "sigmoid_d3"])
 @pytest.mark.parametrize("causal", [True, False])
@@ -28,6 +36,7 @@ def _out(ext, q, k, v, mode, causal, valid=-1):
                                              (256, 257, -1), (256, 448, 385), (128, 1000, -1)])
 def test_eight_wave_blocks_match_four(spline_ops, cuda, mode, causal, heads, seq, valid):
     print(f"blocks {mode} causal {causal} heads {heads} seq {seq} valid {valid}", flush=True)
+    assert _eight_waves(heads, seq) and not _eight_waves(8, seq)
     q, k, v = (t.to(cuda) for t in _inputs(1, heads, heads // 8, seq, seq, d=128)[:3])
     got = _out(spline_ops, q, k, v, mode, causal, valid)
     few = _out(spline_ops, q[:, :, -8:], k[:, :, -1:], v[:, :, -1:], mode, causal, valid)
@@ -55,6 +64,7 @@ def test_rows_past_32_bit_offsets(spline_ops, cuda, d):
 @pytest.mark.parametrize("d,heads,seq", [(64, 6, 1), (64, 4, 200), (128, 4, 129), (128, 512, 33)])
 def test_heads_first_output(spline_ops, cuda, mode, d, heads, seq):
     print(f"heads first {mode} d {d} heads {heads} seq {seq}", flush=True)
+    assert d == 64 or _eight_waves(2 * heads, seq) == (heads == 512)  # batch 2
     q, k, v = (t.to(cuda) for t in _inputs(2, heads, heads // 2, seq, d + seq, d=d)[:3])
     args = (M[mode], 12, True, 1 / math.sqrt(d), 30.0, 0.0)
     out, lse = spline_ops.flash_attn_fwd_bf16(q, k, v, *args)
@@ -129,6 +139,7 @@ def test_wrapper_output_and_gradient_layouts(cuda, own):
 def test_infinite_last_row_of_v(spline_ops, cuda, mode, d, heads, seq):
     print(f"infinite v {mode} d {d} heads {heads} seq {seq}", flush=True)
     q, k, v = (t.to(cuda) for t in _inputs(1, heads, heads, seq, d + seq, d=d)[:3])
+    assert d == 64 or _eight_waves(heads, seq) == (heads == 512)
     v[:, -1, :, 3] = float("inf")
     out = spline_ops.flash_attn_fwd_bf16(q, k, v, M[mode], 12, False, 1 / math.sqrt(d), 30.0, 0.0, -1)[0]
     assert (out[..., 3] == float("inf")).all()

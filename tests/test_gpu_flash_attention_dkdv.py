@@ -1,4 +1,4 @@
-"""dK / dV in 256-key blocks (grids of two rounds and more at head_dim 128)
+"""dK / dV in 256-key blocks (grids that fill the CUs at head_dim 128)
 against the 128- and 64-key blocks that a few of the same heads run in: dS
 is the same to the bit (so is dQ), and the FP32 sums over queries differ in
 order only.  The small grids' results are compared with the float32
@@ -30,15 +30,32 @@ def _agree(got, want):
     return bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2.0 ** -12 * b.abs().max()).all())
 
 
-# 512 blocks of 256 keys: one key, a wave's last key, the block's middle and
-# end, one key into the second block, dS kept (256) or not
+def _wide(heads, seq, causal):
+    """The launcher's rule for 256-key blocks at head_dim 128
+    (dkdv_wide_blocks in flash_attn_bwd.hip), which has to change with it."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = heads * -(-seq // 256)
+    if causal:
+        return blocks >= 2 * cus
+    return 19 * -(-blocks // cus) <= 10 * -(-heads * -(-seq // 128) // cus)
+
+
+# two rounds of 256-key blocks under the mask; without it one round where
+# 128-key blocks take two, or two where they take four (heads per CU).  One key
+# and one wave's keys (without the mask so few never take these blocks), the
+# block's middle and end, one key into its second half and into the second
+# block, dS kept (256, 384, 512) or not
 @pytest.mark.parametrize("mode,grad,route", [("softmax_native", 0, 0), ("softmax_d2", 0, 32), ("softmax_d2", 0, 14),
                                              ("softcap_d4", 1, 0), ("sigmoid_d3", 0, 0)])
-@pytest.mark.parametrize("causal", [True, False])
-@pytest.mark.parametrize("heads,group,seq", [(512, 4, 1), (512, 1, 32), (512, 4, 161), (512, 1, 256), (256, 8, 257),
-                                             (256, 4, 384), (128, 4, 1000)])
-def test_wide_blocks_match_narrow(spline_ops, cuda, mode, grad, route, causal, heads, group, seq):
+@pytest.mark.parametrize("causal,per_cu,group,seq", [
+    (True, 2, 4, 1), (True, 2, 1, 32), (True, 2, 4, 161), (True, 2, 1, 256), (True, 1, 8, 257), (True, 1, 4, 384),
+    (True, 0.5, 4, 1000),
+    (False, 1, 4, 129), (False, 1, 1, 161), (False, 1, 8, 256), (False, 0.5, 4, 257), (False, 0.5, 1, 384),
+    (False, 1, 4, 385), (False, 1, 4, 512), (False, 0.25, 4, 1000)])
+def test_wide_blocks_match_narrow(spline_ops, cuda, mode, grad, route, causal, per_cu, group, seq):
+    heads = int(per_cu * torch.cuda.get_device_properties(0).multi_processor_count)
     print(f"dkdv {mode} route {route} causal {causal} heads {heads} group {group} seq {seq}", flush=True)
+    assert _wide(heads, seq, causal) and not _wide(8, seq, causal)
     t = [x.to(cuda) for x in _inputs(1, heads, heads // group, seq, seq + group)]
     many = _grads(spline_ops, t, mode, grad, causal, route)
     few = _grads(spline_ops, [t[0][:, :, -8:], t[1][:, :, -8 // group:], t[2][:, :, -8 // group:], t[3][:, :, -8:]],
@@ -51,6 +68,7 @@ def test_wide_blocks_match_narrow(spline_ops, cuda, mode, grad, route, causal, h
 
 def test_wide_blocks_rows_past_32_bit_offsets(spline_ops, cuda):
     print("dkdv wide rows", flush=True)
+    assert _wide(512, 9, True)
     t = [x.to(cuda) for x in _inputs(1, 512, 512, 9, 5)]
     want = _grads(spline_ops, t, "softmax_native", 0, True, 0)
     step = (1 << 27) + 8
@@ -84,6 +102,7 @@ def test_infinite_last_row_of_dout(spline_ops, cuda, mode, heads):
     """Queries past the sequence add zeros to dV, not a masked probability
     times the last row's infinity."""
     print(f"infinite dout {mode} heads {heads}", flush=True)
+    assert _wide(heads, 161, False) == (heads == 512)
     t = [x.to(cuda) for x in _inputs(1, heads, heads, 161, 161)]
     t[3][:, -1, :, 3] = float("inf")
     dv = _grads(spline_ops, t, mode, 0, False, 0)[2]
