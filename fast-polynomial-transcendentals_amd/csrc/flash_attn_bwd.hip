@@ -229,10 +229,9 @@ __global__ void __launch_bounds__(256) attn_delta_kernel(const uint16_t* __restr
 }
 
 // ---------------------------------------------------------------------------
-// staging of a 32-row tile, row-major as it arrives.  Thread (pair pr, chunk
-// dc) holds rows 2 pr, 2 pr + 1, BF16 elements 8 dc .. 8 dc + 7; 16 x HD / 8
-// threads move a tile.  The transposed operands (Q^T, dO^T, K^T) are read
-// from the same rows with gfx950's transposing LDS loads.
+// LDS tiles staged through registers, row-major as they arrive.  The
+// transposed operands (Q^T, dO^T, K^T) are read from the same rows with
+// gfx950's transposing LDS loads.
 // ---------------------------------------------------------------------------
 
 // BF16 elements per LDS row.  Each tile is read both by 16-byte row
@@ -243,12 +242,6 @@ template <int HD>
 constexpr int q_row_stride() { return HD + 16; }
 template <int HD>
 constexpr int k_row_stride() { return HD + 24; }
-
-template <int RS>
-__device__ __forceinline__ void store_rows(uint16_t* rows, int pr, int dc, const u32x4_t& a, const u32x4_t& b) {
-    *reinterpret_cast<u32x4_t*>(rows + (2 * pr) * RS + dc * 8) = a;
-    *reinterpret_cast<u32x4_t*>(rows + (2 * pr + 1) * RS + dc * 8) = b;
-}
 
 __device__ __forceinline__ bf16x8_t to_frag(const float (&x)[16], int cc) {
     bf16x8_t f;

@@ -199,7 +199,7 @@ NO_DIVISION = re.compile(r"pt::(pairwise_kernel|pairwise_element_kernel|sincos_t
                          r"sincos_compute_kernel|sincos_f32_kernel|exp2_bf16_kernel|exp2_f32_kernel|b3_f32_kernel|"
                          r"ref_sincos_kernel)\b")
 # sigmoid-attention modes with a score program: B3 (6), B3-D2 (7), BF16 D3-D6 (8-11)
-POLY_ATTENTION = re.compile(r"pt::flash_(fwd|bwd_dkdv|bwd_dq)_kernel<(6|7|8|9|10|11),")
+POLY_ATTENTION = re.compile(r"pt::flash_(fwd|bwd_dkdv|bwd_dkdv256|bwd_dq)_kernel<(6|7|8|9|10|11),")
 
 
 def _polynomial(name: str) -> bool:
@@ -215,7 +215,8 @@ def _polynomial(name: str) -> bool:
 def test_audit_sees_every_family(kernels):
     assert len(kernels) > 900
     for family in ("pairwise_kernel", "packed_fwd_kernel", "sincos_compute_kernel", "rope_apply_kernel",
-                   "flash_fwd_kernel", "flash_bwd_dkdv_kernel", "flash_bwd_dq_kernel", "exp2_bf16_kernel"):
+                   "flash_fwd_kernel", "flash_bwd_dkdv_kernel", "flash_bwd_dkdv256_kernel", "flash_bwd_dq_kernel",
+                   "flash_bwd_dq_ds_kernel", "exp2_bf16_kernel"):
         assert any(f"pt::{family}<" in k for k in kernels), family
     poly = [k for k in kernels if _polynomial(k)]
     assert len(poly) > 500
@@ -280,11 +281,8 @@ def test_no_register_spills_outside_the_measured_exception(metadata):
     waves per SIMD and spill at most a few registers (measured faster than
     the unspilled two-wave form); their instantiations for sequences that are
     not a multiple of 128 (and the softcap D4 one) carry the row guards and
-    spill up to 4 registers / 20 bytes.  No forward kernel spills: the
-    packed FP16 exp2 programs, whose 4-wave head_dim-128 blocks would (both
-    lanes of each packed pair stay live), run 8-wave blocks at head_dim 128
-    whatever the number of query blocks, so those kernels are not built.
-    The softcap dK/dV kernels at head_dim 64 that also store dS for the
+    spill up to 4 registers / 20 bytes.  No forward kernel spills, and none
+    of the 256-key dK/dV and dS-reading dQ kernels.  The softcap dK/dV kernels at head_dim 64 that also store dS for the
     dS-keeping backward spill up to 10 registers / 28 bytes (measured: that
     backward is still 1.1-1.3x the recomputing one)."""
     assert len(metadata) > 900
