@@ -295,11 +295,31 @@ struct FwdShape {
 };
 
 // Waves per SIMD the register allocation is held to: 2 at head_dim 128 (256
-// VGPRs); the head_dim-64 kernels fit three 4-wave blocks per CU (168 VGPRs)
-// except the softcap modes (172 and 175).
+// VGPRs), 3 at head_dim 64 (168), where three 4-wave blocks share a CU.
+template <int HD>
+constexpr int fwd_waves_per_eu() { return HD == 64 ? 3 : 2; }
+
+constexpr bool attn_is_softcap(int mode) { return mode == kAttnSoftcapNative || mode == kAttnSoftcapD4; }
+
+// The kernel's own order of issue (priority while a wave only issues the S
+// MFMAs, LDS reads a fixed number ahead of the products) against the
+// compiler's: the softcap and sigmoid modes at head_dim 64 run faster the
+// latter way (S 4096, 32 heads, causal / not, with the order: hardware sigmoid
+// 106 / 200 us, sigmoid D3 127 / 237, B3-D2 125 / 231; without: 104 / 191, 124 /
+// 221, 123 / 225).
 template <int MODE, int HD>
-constexpr int fwd_waves_per_eu() {
-    return HD == 64 && MODE != kAttnSoftcapD4 && MODE != kAttnSoftcapNative ? 3 : 2;
+constexpr bool fwd_ordered() { return HD != 64 || attn_is_plain_softmax(MODE); }
+
+// Each 16 keys' products right behind their probabilities, which then hold 4
+// VGPRs instead of 16: the polynomial softmax, B3 and softcap D4 at head_dim 64
+// (S 4096, 32 heads, causal / not, against all products behind all
+// probabilities: B3 130 / 236 us against 132 / 236, B3-D2 123 / 225 against 125
+// / 224, while sigmoid D3 loses, 126 / 226 against 124 / 221, and hardware
+// softcap, 168 / 303 against 166 / 299; softcap D4 spills the other way).
+template <int MODE, int HD>
+constexpr bool fwd_fused() {
+    return HD == 64 && (attn_has_exp2_program(MODE) || MODE == kAttnSigmoidB3 || MODE == kAttnSigmoidB3D2 ||
+                        MODE == kAttnSoftcapD4);
 }
 
 // Grid (q_heads, ceil(S / (32 W)), batch), W waves of 32 queries per block:
@@ -312,11 +332,12 @@ constexpr int fwd_waves_per_eu() {
 // a wave with no query at all only stages.
 template <int MODE, int ROUTE, int HD, int W>
 __global__ void __launch_bounds__(64 * W)
-    __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu<MODE, HD>()))) flash_fwd_kernel(AttnParams p) {
+    __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu<HD>()))) flash_fwd_kernel(AttnParams p) {
     using F = FwdShape<HD, W>;
     constexpr int kRing = F::kRing, kRowB = F::kRowB, kTileB = F::kTileB;
     constexpr bool kSigmoid = attn_is_sigmoid(MODE);
     constexpr bool kLate = W == 8;  // the second wave of each SIMD runs half a tile behind
+    constexpr bool kOrdered = fwd_ordered<MODE, HD>(), kFused = fwd_fused<MODE, HD>();
     constexpr int kAheadV = kLate ? kRing - 2 : kRing - 1, kInFlight = kLate ? kRing - 3 : kRing - 2;
     constexpr int kC = HD / 16, kD = HD / 32;
     // K ring, V ring
@@ -406,8 +427,8 @@ __global__ void __launch_bounds__(64 * W)
     f32x16_t s[2];
     auto scores = [&](int i) {
         const uint32_t tile = (uint32_t)(i % kRing * kTileB);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (!kLate) __builtin_amdgcn_s_setprio(1);  // the other blocks keep the VALU busy meanwhile
+        if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!kLate && kOrdered) __builtin_amdgcn_s_setprio(1);  // the other blocks keep the VALU busy meanwhile
         s[0] = s[1] = (f32x16_t){};
 #pragma unroll
         for (int c = 0; c < kC; ++c)
@@ -422,8 +443,8 @@ __global__ void __launch_bounds__(64 * W)
             }
             __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
         }
-        if constexpr (!kLate) __builtin_amdgcn_s_setprio(0);
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!kLate && kOrdered) __builtin_amdgcn_s_setprio(0);
+        if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
     };
     // O^T += V^T P^T of the 16 keys g
     bf16x8_t pf[4];
@@ -432,12 +453,6 @@ __global__ void __launch_bounds__(64 * W)
         for (int dt = 0; dt < kD; ++dt)
             oacc[dt] = mfma32(reader.col_frag(smem + tile + lds_row<HD>(16 * g), dt), pf[g], oacc[dt]);
     };
-    // With independent 4-wave blocks the polynomial programs run faster with
-    // each 16 keys' products right behind their probabilities (head_dim 64,
-    // causal, S 4096, 32 heads: B3 143 against 150 us, D2 at 4 of 12 111
-    // against 114; hardware exp2 101 and softcap 202 against 103 and 208 the
-    // other way).
-    constexpr bool kFused = HD == 64 && (attn_has_exp2_program(MODE) || kSigmoid);
     // probabilities of tile i (masked: it holds the causal diagonal of the
     // wave's queries or keys past the last) as the B operands of P V
     auto probabilities = [&](auto masked_c, int i) {
@@ -457,17 +472,19 @@ __global__ void __launch_bounds__(64 * W)
     // the products of tile i, three fragments read ahead
     auto accumulate = [&](int i) {
         if constexpr (!kFused) {
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int g = 0; g < 4; ++g) accumulate8(kV + (uint32_t)(i % kRing * kTileB), g);
-            __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+            if constexpr (kOrdered) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
-            for (int g = 0; g < 4 * kD - 3; ++g) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                for (int g = 0; g < 4 * kD - 3; ++g) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
-            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -542,11 +559,33 @@ namespace {
 // the ones without a template instantiation take kRouteRuntime
 bool route_supported(int route) { return route >= 4 && route % 2 == 0; }
 
+// LDS that a block asks for beyond its tiles, so that two of them share a CU
+// instead of three: causal softcap at head_dim 64 in grids of two to four
+// blocks a CU, of which each batch element has one a CU and more.  Three to a
+// CU then hold three quarters of the grid and more from the start, so that
+// little is left to even out their unequal lengths; two leave more (the light
+// blocks of what runs first make room for heavy ones).  Hardware softcap /
+// softcap D4, three against two to a CU: S 3072, 32 heads 108 / 136 against 100 /
+// 123 us; S 4096 164 / 205 against 161 / 193; 4 x 1024 63 / 76 against 58 / 68;
+// 3 x 2048, 16 heads 117 / 144 against 90 / 110; worst, 3 x 1280, 65.6 / 77.9
+// against 65.0 / 80.6.  Outside the rule three win: S 4608 192 / 240 against 199
+// / 247; 4 x 1500, 16 heads (0.75 a CU and batch element) 68 / 80 against 80 /
+// 96; S 4096 without the mask 295 / 366 against 306 / 380.
+template <int MODE, int HD, int W>
+unsigned fwd_spare_lds(const AttnParams& prm, int64_t batch) {
+    using F = FwdShape<HD, W>;
+    if (HD != 64 || !attn_is_softcap(MODE) || !prm.causal) return 0;
+    const int64_t cus = device_shape().cus, each = prm.hq * ((prm.seq + F::kBlockQ - 1) / F::kBlockQ);
+    if (each < cus || batch * each <= 2 * cus || batch * each > 4 * cus) return 0;
+    return 160 * 1024 / 3 + 1024 - 2 * F::kRing * F::kTileB;  // a third of the CU's LDS, and more
+}
+
 template <int MODE, int ROUTE, int HD, int W>
 void launch_fwd_shape(const AttnParams& prm, int64_t batch, hipStream_t st) {
     constexpr int kBlockQ = FwdShape<HD, W>::kBlockQ;
     const dim3 grid((unsigned)prm.hq, (unsigned)((prm.seq + kBlockQ - 1) / kBlockQ), (unsigned)batch);
-    hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, HD, W>), grid, dim3(64 * W), 0, st, prm);
+    hipLaunchKernelGGL((flash_fwd_kernel<MODE, ROUTE, HD, W>), grid, dim3(64 * W), (fwd_spare_lds<MODE, HD, W>(prm, batch)),
+                       st, prm);
 }
 
 // Waves per head_dim-128 block.  One 8-wave block per CU stages each tile once

@@ -46,6 +46,29 @@ def test_eight_wave_blocks_match_four(spline_ops, cuda, mode, causal, heads, seq
         assert torch.equal(a[:, -8:], b)
 
 
+def _two_per_cu(batch, heads, seq):
+    """The launcher's rule for causal softcap at head_dim 64 (fwd_spare_lds in
+    flash_attn.hip), which has to change with it."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    each = heads * -(-seq // 128)
+    return each >= cus and 2 * cus < batch * each <= 4 * cus
+
+
+# grids of two to four blocks a CU run two blocks to a CU: two and a half, three
+# and four, one batch element and several
+@pytest.mark.parametrize("mode", ["softcap_native", "softcap_d4"])
+@pytest.mark.parametrize("per_cu,batch,seq", [(0.5, 1, 513), (0.5, 1, 700), (0.5, 1, 1024), (0.25, 3, 500), (1, 4, 33)])
+def test_softcap_grids_of_two_blocks_a_cu(spline_ops, cuda, mode, per_cu, batch, seq):
+    heads = int(per_cu * torch.cuda.get_device_properties(0).multi_processor_count)
+    print(f"two per CU {mode} batch {batch} heads {heads} seq {seq}", flush=True)
+    assert _two_per_cu(batch, heads, seq) and not _two_per_cu(1, 8, seq)
+    q, k, v = (t.to(cuda) for t in _inputs(batch, heads, heads // 8, seq, seq, qmul=4.0, d=64)[:3])
+    got = _out(spline_ops, q, k, v, mode, True)
+    few = _out(spline_ops, q[-1:, :, -8:], k[-1:, :, -1:], v[-1:, :, -1:], mode, True)
+    assert torch.isfinite(got[0]).all()
+    assert torch.equal(got[0][-1:, :, -8:], few[0]) and torch.equal(got[1][-1:, -8:], few[1])
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_rows_past_32_bit_offsets(spline_ops, cuda, d):
     print(f"wide rows d {d}", flush=True)
