@@ -21,8 +21,9 @@
 //  * a block of 4 or 8 waves owns 32 queries per wave, held as the B operand
 //    Q^T (fragments of 8 BF16 per lane);
 //  * 64-key tiles of K and V move from memory straight into rings of LDS
-//    tiles (load_to_lds, swizzled rows), two tiles ahead at head_dim 128; Q
-//    takes the same way once, through the V ring;
+//    tiles (load_to_lds, swizzled rows): K three and V two tiles ahead with 8
+//    waves, both one ahead with 4, both two ahead at head_dim 64; Q takes the
+//    same way once, through the V ring;
 //  * S^T = K Q^T: lane (h, c) of a wave accumulates 16 keys x query c for
 //    each 32-key tile, so every per-query reduction is lane-local plus one
 //    exchange with lane c + 32;
@@ -39,14 +40,13 @@
 //  * causal blocks run from the heaviest query block down.
 //
 // What bounds it: the score program's issue slots next to the matrix cores
-// (head_dim 128, causal, S 4096, 32 query heads: the MFMAs alone take 63 us of
-// the SIMDs), and the power budget: the clock is 2.05 GHz here and 1.8 GHz
-// where MFMAs run back to back.
+// (head_dim 128, causal, S 4096, 32 query heads: 4,160 MFMAs of 32 cycles a
+// SIMD, 65 us of its time at 2.05 GHz), and the power budget: the clock is
+// 2.05 GHz here and 1.8 GHz where MFMAs run back to back.
 #include <hip/hip_runtime.h>
 
 #include "flash_attn.hpp"
 #include "spline_ops_hip.h"
-
 
 namespace pt {
 
@@ -315,7 +315,8 @@ constexpr bool fwd_ordered() { return HD != 64 || attn_is_plain_softmax(MODE); }
 // (S 4096, 32 heads, causal / not, against all products behind all
 // probabilities: B3 130 / 236 us against 132 / 236, B3-D2 123 / 225 against 125
 // / 224, while sigmoid D3 loses, 126 / 226 against 124 / 221, and hardware
-// softcap, 168 / 303 against 166 / 299; softcap D4 spills the other way).
+// softcap, 168 / 303 against 166 / 299; softcap D4 spills the other way, the
+// polynomial softmax is within 3 % either way).
 template <int MODE, int HD>
 constexpr bool fwd_fused() {
     return HD == 64 && (attn_has_exp2_program(MODE) || MODE == kAttnSigmoidB3 || MODE == kAttnSigmoidB3D2 ||
@@ -589,14 +590,32 @@ void launch_fwd_shape(const AttnParams& prm, int64_t batch, hipStream_t st) {
 }
 
 // Waves per head_dim-128 block.  One 8-wave block per CU stages each tile once
-// for 256 queries and is the faster shape where its blocks fill the CUs
-// evenly: an even number of whole rounds (causal blocks are dispatched
-// heaviest first, so two rounds add up to equal loads), or many rounds.
-// Anything else ends in a round that leaves CUs idle, and two 4-wave blocks
-// per CU, half the size, lose less.  Causal, 32 heads, hardware softmax /
-// softcap D4, 8 against 4 waves: S 4096 (two rounds) 151 / 221 against 156 /
-// 238 us; S 6001 (three) 314 / 487 against 299 / 461; S 2048 (one) 65 / 104
-// against 59 / 85.
+// for 256 queries; two 4-wave blocks per CU are half the size and leave less
+// of the chip idle in a round that is not full.  8 waves are taken where their
+// blocks make an even number of whole rounds (causal blocks are dispatched
+// heaviest first, so two rounds add up to equal loads) and from ten rounds on.
+// Time with 4 waves over time with 8, by rounds of 8-wave blocks (32 heads over
+// 8, S = 2048 rounds; hardware softmax / D2 at 4 of 12 / softcap D4 / sigmoid
+// D3):
+//   rounds   causal                       without the mask
+//   1        0.89  0.88  0.81  0.79       1.03  1.04  1.12  1.03
+//   1.5      0.95  0.92  0.96  0.90       0.91  0.89  0.88  0.83
+//   1.75     0.99  1.02  1.07  1.05       1.01  1.03  1.10  1.00
+//   1.88     1.02  1.05  1.09  1.08       1.02  1.03  1.09  1.01
+//   2        0.99  1.04  1.07  1.06       1.01  1.03  1.09  1.01
+//   2.12     0.98  0.98  1.02  0.99       0.93  0.91  0.91  0.85
+//   2.5      0.98  0.95  0.98  0.92       0.94  0.93  0.93  0.88
+//   3        0.98  0.95  0.97  0.92       1.02  1.03  1.07  1.01
+//   4        1.00  1.02  1.04  0.95       1.02  1.03  1.07  0.99
+//   5        0.99  0.98  1.02  0.92       1.02  1.03  1.07  0.99
+//   6        1.01  0.99  1.04  0.96       1.02  1.03  1.06  0.99
+//   10       1.01  1.01  1.04  0.98       1.03  1.02  1.06  1.00
+//   11       1.00  1.00  1.03  0.97       1.05  1.02  1.06  1.00
+// So the rule is on the right side at one round causal, at two, and between
+// whole rounds at a half and less.  It leaves up to 1.12 (softcap) where a
+// second round is nearly full (62 heads, 1.94: softmax 0.96, softcap 1.14) and
+// at odd whole rounds without the mask, and costs the sigmoid modes up to 5 %
+// at four causal rounds and more.
 int fwd_waves(const AttnParams& prm, int64_t batch) {
     const int64_t blocks = batch * prm.hq * ((prm.seq + 255) / 256), cus = device_shape().cus;
     return blocks % (2 * cus) == 0 || blocks >= 10 * cus ? 8 : 4;

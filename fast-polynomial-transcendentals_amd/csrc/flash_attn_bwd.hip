@@ -1186,14 +1186,26 @@ using namespace pt;
 namespace {
 
 // Whether the head_dim-128 dK/dV runs 256-key blocks.  One of them a CU does
-// the work of two 128-key blocks in 0.9 of their time, so it pays where its
-// larger grains still fill the rounds.  Causal (heaviest blocks first, 32
-// heads; 128-key against 256-key blocks, softmax / softcap D4): two rounds
-// and more (S 4096, 382 / 522 against 350 / 490 us), at one and a half the
-// softcap loses (S 3072, 242 / 328 against 232 / 345) and at one both (S 2048,
-// 119 / 159 against 140 / 221).  Without the mask all blocks are alike and
-// whole rounds of both count (one round of 256-key blocks, S 2048: 209 against
-// 187; half a round, S 1000: 53 against 70).
+// the work of two 128-key blocks (four 64-key ones in the sigmoid modes) in
+// 0.9 of their time, so it pays where its larger grains still fill the rounds:
+// causal (heaviest blocks first) from two rounds of 256-key blocks on, without
+// the mask, where all blocks are alike, wherever 128-key blocks take about
+// twice the whole rounds.  Time of the whole backward with the smaller blocks
+// over its time with 256-key ones, by rounds of the latter (32 heads over 8, S
+// = 2048 rounds; hardware softmax / D2 at 4 of 32 / softcap D4 / sigmoid D3; *
+// where the rule takes 256):
+//   rounds   causal                       without the mask
+//   1        0.84  0.78  0.73  0.81       1.12  1.09  1.07  1.13  *
+//   1.5      1.04  1.00  0.97  0.98       0.98  0.92  0.89  0.96
+//   1.75     1.09  1.05  1.03  1.06       1.13  1.08  1.07  1.06  *
+//   1.88     1.09  1.05  1.04  1.07       1.12  1.08  1.07  1.12  *
+//   2        1.10  1.07  1.04  1.08  *    1.11  1.06  1.06  1.12  *
+//   2.12     1.08  1.04  1.02  1.06  *    1.02  0.96  0.93  0.96
+//   2.5      1.07  1.01  0.99  1.05  *    1.03  0.98  0.93  1.04
+//   3        1.06  1.02  0.98  1.06  *    1.11  1.05  1.05  1.13  *
+//   4        1.08  1.06  1.03  1.09  *    1.10  1.04  1.06  1.12  *
+// The causal line could lie at one and three quarters; softcap loses 2 % at
+// two and a half to three.
 bool dkdv_wide_blocks(const AttnBwdParams& prm, int64_t batch) {
     const int64_t cus = device_shape().cus, heads = batch * prm.hq;
     const int64_t blocks = heads * ((prm.seq + DkdvShape::kKeys - 1) / DkdvShape::kKeys);
